@@ -1284,6 +1284,22 @@ struct TbCfg {
 
 constexpr int64_t kTargetBlocks = 1024;
 
+// Launch shape of a one-step launch whose fields (the one read, the one
+// written, the adjoint's f_t) together fit the 256 MiB Infinity Cache: 2
+// rows x 4 waves.  The few-row shape puts more, shorter waves in flight,
+// which is what a launch of a few microseconds waits on, and the written
+// field is read by the next step's launch, so it is stored through the
+// caches (NT stores send it past them) unless the fields are small enough
+// (40 MiB, about the eight L2s) that writing the dirty lines back at the
+// launch's end costs more than it saves.  Ping-pong steps measured, 8 x 2
+// NT / 2 x 4 NT / 2 x 4 cached: FP64 128^3 10.4 / 6.5 / 7.2 us, 192x200x210
+// 34.4 / 31.9 / 22.8, 256^3 63.5 / 54.2 / 40.5, 384^3 (beyond the cache)
+// 166 / 172 / 178; FP32 (4 x 2 NT) 192x200x210 19.2 / 18.1 / 13.1, 256^3
+// 29.9 / 29.8 / 21.9; bf16 384^3 51.6 / 51.4 / 41.9; adjoint with products
+// FP64 120x161x192 33.5 / 27.6 / 25.4, FP32 192x200x210 36.8 / 31.2 / 27.5.
+constexpr int64_t kResidentBytes = 256ll << 20;
+constexpr int64_t kCachedStoreBytes = 40ll << 20;
+
 }  // namespace
 
 // The device's compute units (queried once).
@@ -1403,13 +1419,15 @@ TbCfg tb_default(int bytes, int K) {
 // FDB_ERR_INVALID instead of launching (tuning_error()).
 struct Tuning {
   RowsCfg rows[2][9][9];  // [adj][bytes][fbytes]
+  bool rows_env[2][9][9] = {};  // set by FDB_ROWS_CFG* / FDB_ADJ_CFG_*
   TbCfg tb[9][kMaxTimeBlock + 1];  // [bytes][K]
   bool tb_env[9][kMaxTimeBlock + 1] = {};  // set by FDB_TB_CFG_<bytes>_<K>
   std::string error;
 };
 
 bool rows_shape_ok(const RowsCfg& c) {
-  if (c.chunk < 0 || c.grid < 0 || c.nt != 1) return false;  // non-temporal stores only
+  if (c.chunk < 0 || c.grid < 0 || c.nt < 0 || c.nt > 1) return false;
+  if (c.nt == 0) return c.R == 2 && c.WY == 4;  // cached stores: the resident fields' shape
   for (const auto& s : kRowsShapes)
     if (s[0] == c.R && s[1] == c.WY) return true;
   return false;
@@ -1471,14 +1489,18 @@ Tuning load_tuning() {
   for (int b : sizes) {
     RowsCfg f = rows_default(b, false, 0);
     snprintf(name, sizeof(name), "FDB_ROWS_CFG_%d", b);
-    if (!rows_env(name, f)) rows_env("FDB_ROWS_CFG", f);
-    for (int fb = 0; fb < 9; ++fb) t.rows[0][b][fb] = f;
+    const bool set = rows_env(name, f) || rows_env("FDB_ROWS_CFG", f);
+    for (int fb = 0; fb < 9; ++fb) {
+      t.rows[0][b][fb] = f;
+      t.rows_env[0][b][fb] = set;
+    }
     for (int fb : {0, 8, 4, 2}) {
       RowsCfg a = rows_default(b, true, fb);
       snprintf(name, sizeof(name), "FDB_ADJ_CFG_%d_%d", b, fb);
-      if (!rows_env(name, a)) {
+      t.rows_env[1][b][fb] = rows_env(name, a);
+      if (!t.rows_env[1][b][fb]) {
         snprintf(name, sizeof(name), "FDB_ADJ_CFG_%d", b);
-        rows_env(name, a);
+        t.rows_env[1][b][fb] = rows_env(name, a);
       }
       t.rows[1][b][fb] = a;
     }
@@ -1504,8 +1526,18 @@ const Tuning& tuning() {
   return t;
 }
 
-RowsCfg rows_cfg(int bytes, bool adj, int fbytes = 0) {
-  return tuning().rows[adj ? 1 : 0][bytes][adj ? fbytes : 0];
+// The shape for a step over ntot cells (kResidentBytes: the small fields').
+RowsCfg rows_cfg(int bytes, bool adj, int fbytes, int64_t ntot) {
+  const Tuning& t = tuning();
+  const int a = adj ? 1 : 0, fb = adj ? fbytes : 0;
+  RowsCfg c = t.rows[a][bytes][fb];
+  const int64_t cell = 2 * bytes + fb;
+  if (!t.rows_env[a][bytes][fb] && ntot <= kResidentBytes / cell) {
+    c.R = 2;
+    c.WY = 4;
+    c.nt = ntot <= kCachedStoreBytes / cell ? 1 : 0;
+  }
+  return c;
 }
 
 // Launches the rows kernel for one step (forward: dirs = u, adjoint:
@@ -1515,7 +1547,7 @@ hipError_t rows_dispatch(const Grid3& g, const TS* in, TS* out, const int dirs[3
                          const TF* ft, double* partials, int64_t* nblocks_out, hipStream_t s,
                          bool dry, uint32_t sr_key = 0) {
   using M = typename St<TS>::M;
-  const RowsCfg cfg = rows_cfg((int)sizeof(TS), ADJ, ft ? (int)sizeof(TF) : 0);
+  RowsCfg cfg = rows_cfg((int)sizeof(TS), ADJ, ft ? (int)sizeof(TF) : 0, g.ntot);
   MarchArgs a;
   a.sr_key = sr_key;
   a.n0 = g.n[0];
@@ -1544,19 +1576,28 @@ hipError_t rows_dispatch(const Grid3& g, const TS* in, TS* out, const int dirs[3
     return ((a.n2 + w - 1) / w) * w - a.n2;
   };
   while (vec > 1 && idle(vec / 2) < idle(vec)) vec >>= 1;
-  const int R = cfg.R, WY = cfg.WY;
   a.tiles2 = (a.n2 + 64 * vec - 1) / (64 * vec);
-  a.tiles1 = (a.n1 + (int64_t)WY * R - 1) / ((int64_t)WY * R);
+  auto tiles1 = [&] { return (a.n1 + (int64_t)cfg.WY * cfg.R - 1) / ((int64_t)cfg.WY * cfg.R); };
+  // The products' partial slots stay within 65536 (up to 4 chunks per
+  // tile), the fixed array of the allocation-free entry point: many narrow
+  // tiles keep the taller shape.
+  if (ADJ && ft && a.tiles2 * tiles1() > 16384)
+    cfg = rows_cfg((int)sizeof(TS), ADJ, (int)sizeof(TF), INT64_MAX);
+  const int R = cfg.R, WY = cfg.WY;
+  a.tiles1 = tiles1();
   const int64_t tiles = a.tiles2 * a.tiles1;
   // Axis-0 chunk: an explicit one, or equal chunks for about kTargetBlocks
   // tiles (4 per CU) and up to 4x more, whichever count fills the last
   // round of resident blocks best (occupancy of the kernel launched); each
-  // block takes one tile.
+  // block takes one tile.  A grid with too few tiles for that takes one
+  // plane per block (one march through all the planes of a 32x24x40 grid
+  // ran 40 us, one plane per block 3.9).
   hipError_t result = hipErrorInvalidValue;
   auto go = [&](auto kern, int W) {
     int64_t chunk = cfg.chunk;
     if (chunk <= 0) {
-      const int64_t lo = std::max<int64_t>(1, (kTargetBlocks + tiles / 2) / tiles);
+      const int64_t lo =
+          std::min(a.n0, std::max<int64_t>(1, (kTargetBlocks + tiles / 2) / tiles));
       const int64_t nch =
           march_chunks(tiles, a.n0, 1, resident_blocks(kern, 64 * W), lo, 4 * lo, false);
       chunk = (a.n0 + nch - 1) / nch;
@@ -1592,6 +1633,7 @@ hipError_t rows_dispatch(const Grid3& g, const TS* in, TS* out, const int dirs[3
   FDB_ROWS_V(4, 4, true)
   FDB_ROWS_V(8, 1, true)
   FDB_ROWS_V(2, 4, true)
+  FDB_ROWS_V(2, 4, false)
   FDB_ROWS_V(2, 8, true)
   FDB_ROWS_V(2, 2, true)
   FDB_ROWS_V(1, 8, true)
