@@ -165,6 +165,7 @@ struct fdb_upwind {
   uint64_t steps_done = 0;  // steps advanced since creation or set_seed
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   void* stage = nullptr;  // pinned host staging
+  char* fold = nullptr;   // device scratch of the exact fold (first checksum on)
 };
 
 namespace {
@@ -176,6 +177,7 @@ int release(fdb_upwind* h) {
     if (b) (void)hipFree(b);
   if (h->partials) (void)hipFree(h->partials);
   if (h->stage) (void)hipHostFree(h->stage);
+  if (h->fold) (void)hipFree(h->fold);
   if (h->ev0) (void)hipEventDestroy(h->ev0);
   if (h->ev1) (void)hipEventDestroy(h->ev1);
   if (h->stream) (void)hipStreamDestroy(h->stream);
@@ -198,6 +200,24 @@ int for_each_chunk(fdb_upwind* h, Fn fn) {
     h_convert(h->dtype, h->stage, FDB_F64, wide.data(), cnt);
     fn(wide.data(), cnt, i0);
   }
+  return FDB_OK;
+}
+
+// The sequential fold of the field (squares: of its squared distances from
+// mean) on the device, where the field is large enough and its scratch can
+// be had; *done tells whether *out was set (the caller folds otherwise).
+int fold_field(fdb_upwind* h, bool squares, double mean, double* out, bool* done) {
+  *done = false;
+  if (h->ntot < fdb::kFoldMinValues) return FDB_OK;
+  const fdb::FoldPlan p = fdb::fold_plan(h->ntot);
+  if (p.host_bytes > kStageBytes) return FDB_OK;
+  if (!h->fold && hipMalloc((void**)&h->fold, p.dev_bytes) != hipSuccess) {
+    (void)hipGetLastError();  // no room for the scratch
+    h->fold = nullptr;
+    return FDB_OK;
+  }
+  FDB_HIP(fdb::fold_exact(h->dtype, h->buf[h->cur], p, squares, mean, h->fold, (char*)h->stage,
+                          h->stream, out, done));
   return FDB_OK;
 }
 
@@ -301,7 +321,11 @@ int fdb_upwind_advect_timed(fdb_upwind_t* h, int num_time_steps, double delta_ti
 
 int fdb_upwind_checksum(fdb_upwind_t* h, double* out) {
   if (!h || !out) return fail(FDB_ERR_INVALID, "checksum: null argument");
-  double s = 0.0;  // std::accumulate(f.begin(), f.end(), 0.0), upwind.cxx:92
+  // std::accumulate(f.begin(), f.end(), 0.0), upwind.cxx:92
+  bool done = false;
+  if (int rc = fold_field(h, false, 0.0, out, &done)) return rc;
+  if (done) return FDB_OK;
+  double s = 0.0;
   int rc = for_each_chunk(h, [&](const double* f, uint64_t n, uint64_t) {
     for (uint64_t i = 0; i < n; ++i) s = s + f[i];
   });
@@ -316,13 +340,18 @@ int fdb_upwind_std(fdb_upwind_t* h, double* out) {
   if (int rc = fdb_upwind_checksum(h, &cs)) return rc;
   const double mean = cs / (double)h->ntot;  // upwind.cxx:96
   double res = 0;
-  int rc = for_each_chunk(h, [&](const double* f, uint64_t n, uint64_t) {
-    for (uint64_t i = 0; i < n; ++i) {
-      const double d = f[i] - mean;
-      res += d * d;
-    }
-  });
-  if (rc) return rc;
+  bool done = false;
+  if (int rc = fold_field(h, true, mean, &res, &done)) return rc;
+  if (!done) {
+    res = 0;
+    int rc = for_each_chunk(h, [&](const double* f, uint64_t n, uint64_t) {
+      for (uint64_t i = 0; i < n; ++i) {
+        const double d = f[i] - mean;
+        res += d * d;
+      }
+    });
+    if (rc) return rc;
+  }
   *out = std::sqrt(res / (double)h->ntot);  // upwind.cxx:102
   return FDB_OK;
 }

@@ -23,6 +23,8 @@ struct fdb_filter {
   bool out_is_in = false;  // after copyOutToIn the output equals the input
   hipStream_t s = nullptr;
   hipEvent_t e0 = nullptr, e1 = nullptr;
+  char* fold_dev = nullptr;   // scratch of the exact fold (first checksum on)
+  char* fold_host = nullptr;  // its pinned host side
 };
 
 namespace {
@@ -62,6 +64,8 @@ void free_filter(fdb_filter* h) {
   if (h->s) (void)hipStreamSynchronize(h->s);
   for (double* b : h->buf)
     if (b) (void)hipFree(b);
+  if (h->fold_dev) (void)hipFree(h->fold_dev);
+  if (h->fold_host) (void)hipHostFree(h->fold_host);
   if (h->e0) (void)hipEventDestroy(h->e0);
   if (h->e1) (void)hipEventDestroy(h->e1);
   if (h->s) (void)hipStreamDestroy(h->s);
@@ -228,7 +232,24 @@ int fdb_filter_checksum(fdb_filter_t* h, int which, double* out) {
   if (!h || !out || (which != 0 && which != 1))
     return ffail(FDB_ERR_INVALID, "filter_checksum: bad argument");
   const double* src = which == 0 ? h->buf[h->in] : out_buf(h);
-  // localSum += data[i] in order (Filter.cpp:470-480), chunk by chunk.
+  // localSum += data[i] in order (Filter.cpp:470-480): on the device where
+  // the field is large enough and the scratch can be had, else chunk by
+  // chunk on the host.
+  if ((uint64_t)h->g.ntot >= fdb::kFoldMinValues) {
+    const fdb::FoldPlan p = fdb::fold_plan((uint64_t)h->g.ntot);
+    if (!h->fold_dev && hipMalloc((void**)&h->fold_dev, p.dev_bytes) != hipSuccess)
+      h->fold_dev = nullptr;
+    if (!h->fold_host && hipHostMalloc((void**)&h->fold_host, p.host_bytes) != hipSuccess)
+      h->fold_host = nullptr;
+    if (h->fold_dev && h->fold_host) {
+      bool done = false;
+      FLT_HIP(fdb::fold_exact(FDB_F64, src, p, false, 0.0, h->fold_dev, h->fold_host, h->s, out,
+                              &done));
+      if (done) return FDB_OK;
+    } else {
+      (void)hipGetLastError();
+    }
+  }
   const uint64_t chunk = (uint64_t)1 << 22;
   std::vector<double> tmp((size_t)std::min<uint64_t>(chunk, (uint64_t)h->g.ntot));
   double sum = 0;

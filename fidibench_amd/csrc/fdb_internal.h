@@ -203,6 +203,37 @@ hipError_t launch_misfit(int f_dtype, const void* f, const void* target, uint64_
                          int lam_dtype, void* lam, double* partials, double* out2,
                          hipStream_t s);
 
+// ---- exact sequential left fold on the device (fdb_fold.hip)
+
+// What one chunk of consecutive values does to the running sum s: nothing
+// (all zeros); in the binade 2^ex of sign neg, adds d0 or d1 (by the parity
+// of its 53-bit integer significand) with every value on the way within
+// [lo, hi] of the start; or unknown, its values copied to slot (-1: not).
+enum { kFoldZero = 0, kFoldMapped = 1, kFoldRaw = 2 };
+struct FoldRec {
+  double d0, d1, lo, hi;
+  int ex, neg, kind, slot;
+};
+struct FoldPlan {
+  uint64_t n, chunk, nchunks, slots;
+  size_t rec_off, gather_off, host_bytes, dev_bytes;
+};
+FoldPlan fold_plan(uint64_t n);
+// Fields below this are folded on the host: the launches and copies of the
+// device fold take about 30 us, the host's copy and dependent additions as
+// long at 32768 values.
+constexpr uint64_t kFoldMinValues = 65536;
+// s = +0; for each value (squares: its squared distance from mean, rounded
+// per operation) s = s + value, in order, with exactly that loop's bits.
+// dev: dev_bytes of device memory; host: host_bytes, pinned for speed.
+// Blocks.  *done = false (and no error) where the field has too many chunks
+// that no map covers: the caller then folds it value by value.
+hipError_t fold_exact(int dtype, const void* x, const FoldPlan& p, bool squares, double mean,
+                      char* dev, char* host, hipStream_t s, double* out, bool* done);
+// The host's step over one chunk of cnt values (vals: the copied chunks of
+// `chunk` values each); false where the record does not apply to *s.
+bool fold_step(const FoldRec& r, const double* vals, uint64_t chunk, uint64_t cnt, double* s);
+
 // Synthetic initial field (see fdb_init_kind).  params are copied by value.
 hipError_t launch_init(int dtype, const Grid3& g, const double* len, int kind,
                        const double* params, int nparams, uint64_t seed, void* f, hipStream_t s);

@@ -1,0 +1,88 @@
+"""checksum() and std() of fields folded on the device against the
+sequential loop, bit for bit: values that round at every addition, ties
+(single-precision values in a double sum), both signs with the sum passing
+through zero and through binades, zeros, values far apart in magnitude,
+values that are not finite, and sizes around the device path's first one
+and its chunks of 2048."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _fields(n):
+    r = np.random.default_rng(n)
+    u = r.random(n)
+    sign = np.where(r.random(n) < 0.5, -1.0, 1.0)
+    ball = (np.arange(n) % 977 < 300).astype(float)
+    spike = np.zeros(n)
+    spike[0], spike[n // 2], spike[-1] = 1.0, 1e-320, -2.5
+    nan, inf = u.copy(), u.copy()
+    nan[n // 3], inf[n // 2], inf[-1] = np.nan, np.inf, -np.inf
+    return {
+        "positive": u,
+        "noisy_ball": ball + 0.01 * u,
+        "ties": r.random(n, dtype=np.float32).astype(np.float64) * 0.01,
+        "halves": np.where(r.random(n) < 0.5, 0.5, 1.5) * 2.0 ** -38 + np.where(
+            np.arange(n) == 0, 2.0 ** 15, 0.0),
+        "both_signs": u * sign,
+        "negative": -u,
+        "cancel": np.concatenate([u[: n // 2], -u[: n - n // 2]]),
+        "scales": sign * u * 2.0 ** r.integers(-300, 300, n),
+        "spike": spike,
+        "zeros": np.zeros(n) * sign,
+        "tiny": u * 5e-324 * 100,
+        "nan": nan,
+        "inf": inf,
+    }
+
+
+@pytest.mark.parametrize("n", [65535, 65536, 65537, 129 * 2048 - 1, 300 * 2048 + 5])
+def test_folds_equal_the_sequential_loop(oracle, n):
+    from fidibench_amd import Upwind
+    with np.errstate(all="ignore"):
+        for name, f in _fields(n).items():
+            with Upwind((1.0,), (1.0,), (n,)) as up:
+                up.set_field(f)
+                for got, want in ((up.checksum(), oracle.checksum(f)), (up.std(), oracle.std(f))):
+                    same = np.float64(got).tobytes() == np.float64(want).tobytes()
+                    assert same or (np.isnan(got) and np.isnan(want)), (name, n, got, want)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_folds_of_narrow_storage(oracle, dtype):
+    from fidibench_amd import Upwind
+    shape = (61, 70, 83)
+    f = oracle.uniform(shape, -0.2, 1.0, seed=9)
+    with Upwind((1.0, 1.0, 1.0), (1.0, 1.0, 1.0), shape, dtype=dtype) as up:
+        up.set_field(f)
+        wide = up.get_field("f64")
+        assert up.checksum() == oracle.checksum(wide)
+        assert up.std() == oracle.std(wide)
+
+
+def test_fold_of_a_long_field(oracle):
+    """Chunks longer than one tile: 2^25 + 3 values fold in chunks of 4096."""
+    from fidibench_amd import Upwind
+    n = 2 ** 25 + 3
+    f = oracle.uniform((n,), 0.0, 1.0, seed=3)
+    with Upwind((1.0,), (1.0,), (n,)) as up:
+        up.set_field(f)
+        assert up.checksum() == oracle.checksum(f)
+
+
+def test_filter_checksums(oracle):
+    from fidibench_amd import Filter
+    dims = (300, 257)
+    rng = np.random.default_rng(4)
+    f = rng.standard_normal(dims)
+    flt = Filter(dims, [0.0, 0.0], [1.0, 1.0], {(0, 0): 0.6, (1, 0): 0.1, (0, -1): 0.3})
+    flt.setInData(f)
+    flt.applyFilter()
+    out = flt.get_data("output").ravel(order="F")
+    assert flt.computeCheckSum("output") == oracle.checksum(np.ascontiguousarray(out))
+    assert flt.computeCheckSum("input") == oracle.checksum(
+        np.ascontiguousarray(f.ravel(order="F")))
+    flt.close()
