@@ -640,7 +640,7 @@ int fdb_plan_passes(int ndims, const uint64_t* num_cells, const double* velocity
     left -= k;
     while (k > 0) {  // the launches of one pass: deepest supported depth first
       int K = 1;
-      for (int c : {8, 7, 6, 4, 3, 2})
+      for (int c : {8, 7, 6, 5, 4, 3, 2})
         if (c <= k && fdb::fused_pass_supported(dtype, g, c)) {
           K = c;
           break;

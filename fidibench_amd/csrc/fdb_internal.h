@@ -85,6 +85,16 @@ hipError_t launch_fused_pass(int dtype, const Grid3& g, const void* src, void* d
 // (FDB_F64, FDB_F32, FDB_BF16, FDB_BF16_SR) and shape in one launch.
 bool fused_pass_supported(int dtype, const Grid3& g, int k);
 
+// A 2-D problem (axes 1 and 2): its fused passes are plane_kernel's
+// (fdb_plane.hip), of 2..8 steps for FP64, FP32 and bf16 round to nearest.
+inline bool is_plane(const Grid3& g) { return !g.act[0] && g.act[1] && g.act[2]; }
+bool plane_pass_supported(int dtype, const Grid3& g, int k);
+// hipErrorNotSupported unless plane_pass_supported; src is only read.
+hipError_t launch_plane_pass(int dtype, const Grid3& g, const void* src, void* dst, int k,
+                             hipStream_t s);
+// Modelled time (us) of one k-step launch over the 2-D grid g.
+float plane_pass_us(int dtype, const Grid3& g, int k);
+
 // Steps of the next launch when `left` (>= 1) steps remain and at most
 // `cap` may be fused: the first pass of the least-time split of `left`
 // into one-step launches and supported fused passes (1 = a one-step

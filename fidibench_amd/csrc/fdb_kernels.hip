@@ -1645,7 +1645,8 @@ hipError_t rows_dispatch(const Grid3& g, const TS* in, TS* out, const int dirs[3
 // Temporally blocked pass: K steps in one launch.  Returns
 // hipErrorNotSupported when the shape does not fit (the caller then runs
 // one-step launches): all three axes present (an absent axis has no term
-// at all, which a fused pass would not reproduce for Inf/NaN values).
+// at all, which a fused pass would not reproduce for Inf/NaN values; 2-D
+// problems have passes of their own, launch_plane_pass).
 // Launch shape (rows per wave, waves per block, target tiles per launch;
 // 0 = chunk count from the kernel's occupancy, below): sweeps at 512^3
 // and 1024^3 on MI355X, all bit-exact, gave 9 rows x 8 waves at K >= 6
@@ -1909,6 +1910,7 @@ bool make_grid(int ndims, const uint64_t* n, const double* v, const double* len,
 
 bool fused_pass_supported(int dtype, const Grid3& g, int k) {
   if (k < 2 || k > kMaxTimeBlock) return false;
+  if (is_plane(g)) return plane_pass_supported(dtype, g, k);
   if (dtype != FDB_F64 && dtype != FDB_F32 && dtype != FDB_BF16 && dtype != FDB_BF16_SR)
     return false;
   const int bytes = (int)dtype_size(dtype);
@@ -2014,6 +2016,11 @@ PassCosts pass_costs(int dtype, const Grid3& g) {
   const float* tab = kPassUs[row];
   const double cells = (double)g.ntot / (512.0 * 512.0 * 512.0);
   PassCosts c{};
+  if (is_plane(g)) {
+    for (int k = 1; k <= kMaxTimeBlock; ++k)
+      if (k == 1 || plane_pass_supported(dtype, g, k)) c.us[k] = plane_pass_us(dtype, g, k);
+    return c;
+  }
   if (cells < 1.0) {
     // Between the measured sizes i and i + 1 (side^3 cells each).
     const double lc = std::log((double)g.ntot);
@@ -2112,6 +2119,8 @@ uint32_t sr_step_key(uint64_t seed, uint64_t step) {
 hipError_t launch_fused_pass(int dtype, const Grid3& g, const void* src, void* dst, int k,
                              hipStream_t s, void* const* levels, uint64_t step0, uint64_t seed) {
   if (k < 2 || src == dst) return hipErrorNotSupported;
+  if (is_plane(g))
+    return levels ? hipErrorNotSupported : launch_plane_pass(dtype, g, src, dst, k, s);
   switch (dtype) {
     case FDB_F64: return tb_dispatch<double>(g, (const double*)src, (double*)dst, k, s, levels);
     case FDB_F32: return tb_dispatch<float>(g, (const float*)src, (float*)dst, k, s, levels);
@@ -2139,20 +2148,10 @@ hipError_t launch_advect_pass(int dtype, const Grid3& g, void* const bufs[2], in
     void* dst = bufs[1 - *cur];
     int done = 0;
     // Temporally blocked pass with the deepest supported K <= left.
-    for (int K : {8, 7, 6, 4, 3, 2}) {
+    for (int K : {8, 7, 6, 5, 4, 3, 2}) {
       if (K > left) continue;
-      switch (dtype) {
-        case FDB_F64: err = tb_dispatch<double>(g, (const double*)src, (double*)dst, K, s); break;
-        case FDB_F32: err = tb_dispatch<float>(g, (const float*)src, (float*)dst, K, s); break;
-        case FDB_BF16:
-          err = tb_dispatch<uint16_t>(g, (const uint16_t*)src, (uint16_t*)dst, K, s);
-          break;
-        // Stochastic rounding: the bits of step stepno + l at level l.
-        case FDB_BF16_SR:
-          err = launch_fused_pass(dtype, g, src, dst, K, s, nullptr, stepno, seed);
-          break;
-        default: return hipErrorInvalidValue;
-      }
+      // (Stochastic rounding: the bits of step stepno + l at level l.)
+      err = launch_fused_pass(dtype, g, src, dst, K, s, nullptr, stepno, seed);
       if (err == hipSuccess) {
         done = K;
         break;
