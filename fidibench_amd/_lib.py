@@ -58,6 +58,7 @@ SIGNATURES = {
                             C.POINTER(_i)]),
     "fdb_advect_dev_seeded": (_i, [_i, _u64p, _dp, _dp, C.c_double, _i, _vp, _vp, _i, _i,
                                    C.c_uint64, C.c_uint64, _vp, C.POINTER(_i)]),
+    "fdb_advect_from_dev": (_i, [_i, _u64p, _dp, _dp, C.c_double, _i, _vp, _vp, _vp, _i, _vp]),
     "fdb_plan_passes": (_i, [_i, _u64p, _dp, _dp, C.c_double, _i, _i, _i, C.POINTER(_i), _i,
                              C.POINTER(_i)]),
     "fdb_adjoint_step_dev": (_i, [_i, _u64p, _dp, _dp, C.c_double, _i, _vp, _vp, _i, _vp, _vp,
@@ -68,6 +69,9 @@ SIGNATURES = {
     "fdb_misfit_dev": (_i, [_i, _vp, _vp, C.c_uint64, _i, _vp, _dp, _vp]),
     "fdb_tape_create": (_i, [_i, _u64p, _dp, _dp, C.c_double, _i, _i, _i, C.c_uint64,
                              C.POINTER(_vp)]),
+    "fdb_tape_create_in": (_i, [_i, _u64p, _dp, _dp, C.c_double, _i, _i, _i, C.c_uint64, _i,
+                                C.POINTER(_vp), C.POINTER(C.c_uint64)]),
+    "fdb_tape_set_workspace": (_i, [_vp, _vp, C.c_uint64]),
     "fdb_tape_forward": (_i, [_vp, _vp, _vp, _vp]),
     "fdb_tape_backward": (_i, [_vp, _vp, _vp, _dp, _vp]),
     "fdb_tape_stats": (_i, [_vp, C.POINTER(_i), C.POINTER(C.c_int64), C.POINTER(C.c_int64)]),

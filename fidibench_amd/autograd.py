@@ -36,6 +36,12 @@ def _stream() -> int:
     return torch.cuda.current_stream().cuda_stream
 
 
+# A checkpointed tape whose states take more than this allocates them itself
+# and gives them back to the device when it closes; smaller ones lie in
+# torch memory, whose cache keeps them for the next tape.
+_WORKSPACE_MAX = 4 << 30
+
+
 class Tape:
     """Owner of one fdb_tape_t (checkpoint storage for one forward/backward)."""
 
@@ -45,7 +51,10 @@ class Tape:
         self.shape = tuple(int(x) for x in shape)
         self.ndims = len(self.shape)
         self.f_dtype, self.lam_dtype = f_dtype, lam_dtype
-        h = C.c_void_p()
+        self.method = method
+        self._f0 = None
+        self._ws = None  # "checkpoint": the states' torch memory
+        h, need = C.c_void_p(), C.c_uint64()
         if method == "shift":
             # No snapshots in this method: ask for the fixed working set only
             # (initial state, two working buffers, one adjoint buffer).
@@ -54,23 +63,51 @@ class Tape:
                 ntot *= n
             fixed = ntot * (3 * L.ITEMSIZE[f_dtype] + L.ITEMSIZE[lam_dtype])
             max_bytes = min(int(max_bytes), fixed)
-        L.check(L.lib().fdb_tape_create(self.ndims, L.u64s(self.shape), L.dbls(velocity),
-                                        L.dbls(lengths), float(dt), int(nsteps), f_dtype,
-                                        lam_dtype, int(max_bytes), C.byref(h)))
-        self._h = h
-        self.method = method
-        L.check(L.lib().fdb_tape_set_method(h, L.GRAD_METHODS[method]))
-        self._f0 = None
+        args = (self.ndims, L.u64s(self.shape), L.dbls(velocity), L.dbls(lengths), float(dt),
+                int(nsteps), f_dtype, lam_dtype, int(max_bytes))
+        L.check(L.lib().fdb_tape_create_in(*args, L.GRAD_METHODS[method], C.byref(h),
+                                           C.byref(need)))
+        self._h, self._need = h, need.value
+        if method == "checkpoint":
+            if self._need > _WORKSPACE_MAX:
+                self.close()
+                h, self._need = C.c_void_p(), 0
+                L.check(L.lib().fdb_tape_create(*args, C.byref(h)))
+                self._h = h
+            else:
+                self._ws = self._workspace()
+                self._set_workspace(self._ws)
+
+    def _workspace(self) -> torch.Tensor:
+        try:
+            return torch.empty(self._need, dtype=torch.uint8, device="cuda")
+        except torch.cuda.OutOfMemoryError as e:
+            raise L.FdbError(L.ERR_NOMEM, str(e)) from None
+
+    def _set_workspace(self, ws) -> None:
+        L.check(L.lib().fdb_tape_set_workspace(self._h, None if ws is None else ws.data_ptr(),
+                                               self._need))
+
+    def _call(self, fn, *args) -> None:
+        """fn(tape, *args) on the current stream; "shift" tapes hold scratch
+        for this call only (it returns with its work done)."""
+        if self.method == "shift":
+            ws = self._workspace()
+            self._set_workspace(ws)
+        try:
+            L.check(fn(self._h, *args, _stream()))
+        finally:
+            if self.method == "shift":
+                self._set_workspace(None)
 
     def forward(self, f0: torch.Tensor, fT: torch.Tensor) -> None:
-        L.check(L.lib().fdb_tape_forward(self._h, f0.data_ptr(), fT.data_ptr(), _stream()))
+        self._call(L.lib().fdb_tape_forward, f0.data_ptr(), fT.data_ptr())
         # "shift" reads f0 again in backward: keep the tensor alive until then.
         self._f0 = f0 if self.method == "shift" else None
 
     def backward(self, lamT: torch.Tensor, lam0: torch.Tensor) -> list:
         gv = (C.c_double * 3)()
-        L.check(L.lib().fdb_tape_backward(self._h, lamT.data_ptr(), lam0.data_ptr(), gv,
-                                          _stream()))
+        self._call(L.lib().fdb_tape_backward, lamT.data_ptr(), lam0.data_ptr(), gv)
         return [gv[i] for i in range(self.ndims)]
 
     def set_time_block(self, k: int) -> None:
@@ -88,6 +125,7 @@ class Tape:
             L.lib().fdb_tape_destroy(self._h)
             self._h = C.c_void_p()
         self._f0 = None
+        self._ws = None
 
     def __del__(self):
         try:
@@ -111,15 +149,14 @@ class UpwindAdvect(torch.autograd.Function):
         v = [float(x) for x in velocity.detach().double().cpu().reshape(-1).tolist()]
         f0c = f0.detach().contiguous()
         if not any(ctx.needs_input_grad[:2]):
-            # No gradient wanted: plain ping-pong advect, no checkpoints.
-            a = f0c.clone()
-            b = torch.empty_like(a)
-            res = C.c_int()
-            L.check(L.lib().fdb_advect_dev(a.dim(), L.u64s(a.shape), L.dbls(v), L.dbls(lengths),
-                                           float(dt), f_dtype, a.data_ptr(), b.data_ptr(),
-                                           int(nsteps), 1, _stream(), C.byref(res)))
+            # No gradient wanted: the planner's passes, no checkpoints.
+            fT, tmp = torch.empty_like(f0c), torch.empty_like(f0c)
+            L.check(L.lib().fdb_advect_from_dev(fT.dim(), L.u64s(fT.shape), L.dbls(v),
+                                                L.dbls(lengths), float(dt), f_dtype,
+                                                f0c.data_ptr(), fT.data_ptr(), tmp.data_ptr(),
+                                                int(nsteps), _stream()))
             ctx.tape = None
-            return b if res.value else a
+            return fT
         budget = max_bytes if max_bytes is not None else default_budget()
         tape = Tape(f0c.shape, v, lengths, dt, nsteps, f_dtype, lam, budget, method=method)
         fT = torch.empty_like(f0c)

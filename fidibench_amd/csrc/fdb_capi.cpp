@@ -621,6 +621,26 @@ int fdb_advect_dev(int ndims, const uint64_t* num_cells, const double* velocity,
                                nsteps, time_block, 0, 0, stream, result_in_b);
 }
 
+int fdb_advect_from_dev(int ndims, const uint64_t* num_cells, const double* velocity,
+                        const double* lengths, double delta_time, int dtype, const void* src,
+                        void* dst, void* tmp, int nsteps, void* stream) {
+  fdb::Grid3 g;
+  if (!fdb::make_grid(ndims, num_cells, velocity, lengths, delta_time, &g))
+    return fail(FDB_ERR_INVALID, "advect_from_dev: invalid geometry");
+  if (!valid_dtype(dtype)) return fail(FDB_ERR_INVALID, "advect_from_dev: unknown dtype");
+  if (!src || !dst || !tmp || src == dst || src == tmp || dst == tmp)
+    return fail(FDB_ERR_INVALID, "advect_from_dev: need three distinct buffers");
+  if (int rc = check_tuning()) return rc;
+  if (nsteps <= 0) {
+    FDB_HIP(hipMemcpyAsync(dst, src, (size_t)g.ntot * fdb::dtype_size(dtype),
+                           hipMemcpyDeviceToDevice, (hipStream_t)stream));
+    return FDB_OK;
+  }
+  FDB_HIP(fdb::launch_planned_steps(dtype, g, src, dst, tmp, nsteps, fdb::kMaxTimeBlock,
+                                    (hipStream_t)stream, 0, 0));
+  return FDB_OK;
+}
+
 int fdb_plan_passes(int ndims, const uint64_t* num_cells, const double* velocity,
                     const double* lengths, double delta_time, int dtype, int nsteps,
                     int time_block, int* ks, int max_ks, int* count) {

@@ -101,6 +101,13 @@ float plane_pass_us(int dtype, const Grid3& g, int k);
 // launch).  Every split gives the same results.
 int plan_pass(int dtype, const Grid3& g, int left, int cap);
 
+// nsteps steps from src (only read) into dst by the planner's passes of at
+// most `cap` steps, alternating between dst and tmp (three distinct
+// buffers; tmp may be null where one pass suffices).  Stochastic rounding:
+// steps step0, step0 + 1, ... of a run seeded `seed`.
+hipError_t launch_planned_steps(int dtype, const Grid3& g, const void* src, void* dst, void* tmp,
+                                int nsteps, int cap, hipStream_t s, uint64_t step0, uint64_t seed);
+
 // The storage layout of a dtype (FDB_BF16_SR is stored as FDB_BF16).
 inline int storage_dtype(int dtype) { return dtype == 3 ? 2 : dtype; }
 

@@ -15,6 +15,7 @@
 
 #include <cmath>
 #include <mutex>
+#include <vector>
 
 #include "fdb_internal.h"
 #include "../../include/fidibench_amd/fdb_upwind.h"
@@ -2177,6 +2178,28 @@ hipError_t launch_advect_pass(int dtype, const Grid3& g, void* const bufs[2], in
     ++n;
   }
   if (launches) *launches = n;
+  return hipSuccess;
+}
+
+hipError_t launch_planned_steps(int dtype, const Grid3& g, const void* src, void* dst, void* tmp,
+                                int nsteps, int cap, hipStream_t s, uint64_t step0,
+                                uint64_t seed) {
+  std::vector<int> ks;
+  for (int left = nsteps; left > 0; left -= ks.back())
+    ks.push_back(plan_pass(dtype, g, left, cap));
+  const void* from = src;
+  for (size_t i = 0; i < ks.size(); ++i) {
+    void* to = (ks.size() - 1 - i) % 2 == 0 ? dst : tmp;  // the last one lands in dst
+    if (!to || to == from) return hipErrorInvalidValue;
+    void* const pair[2] = {const_cast<void*>(from), to};
+    int cur = 0;
+    const hipError_t err =
+        ks[i] > 1 ? launch_fused_pass(dtype, g, from, to, ks[i], s, nullptr, step0, seed)
+                  : launch_advect_pass(dtype, g, pair, &cur, 1, s, nullptr, step0, seed);
+    if (err != hipSuccess) return err;
+    from = to;
+    step0 += (uint64_t)ks[i];
+  }
   return hipSuccess;
 }
 

@@ -142,6 +142,11 @@ struct fdb_tape {
   int method = FDB_GRAD_CHECKPOINT;
   bool slots_ready = false;    // snapshot slots allocated (released by FDB_GRAD_SHIFT)
   const void* f0_ref = nullptr;  // FDB_GRAD_SHIFT: the caller's f0
+  // fdb_tape_create_in: the buffers above lie in the caller's workspace
+  // (set_workspace), which the tape neither allocates nor frees.
+  bool external = false;
+  bool ws_set = false;
+  bool partials_own = true;  // partials came from hipMalloc
 };
 
 namespace {
@@ -158,6 +163,11 @@ namespace {
 
 void tape_free(fdb_tape* t) {
   if (!t) return;
+  if (t->external) {  // (its calls return with their work done)
+    if (t->partials && t->partials_own) (void)hipFree(t->partials);
+    delete t;
+    return;
+  }
   (void)hipDeviceSynchronize();
   if (t->base) (void)hipFree(t->base);
   for (void* s : t->slots) (void)hipFree(s);
@@ -167,6 +177,18 @@ void tape_free(fdb_tape* t) {
   if (t->partials) (void)hipFree(t->partials);
   if (t->acc) (void)hipFree(t->acc);
   delete t;
+}
+
+// Layout of a caller's workspace: the accumulator, the partial sums (more
+// than this many bytes come from hipMalloc), then whole fields at 256-byte
+// steps.
+constexpr uint64_t kWsAcc = 256;
+constexpr uint64_t kWsPartials = 1u << 20;
+uint64_t ws_align(uint64_t b) { return (b + 255) / 256 * 256; }
+uint64_t ws_bytes(const fdb_tape* t) {
+  const uint64_t f = ws_align(t->fbytes), l = ws_align(t->lbytes);
+  if (t->method == FDB_GRAD_SHIFT) return kWsAcc + kWsPartials + std::max(f, l);
+  return kWsAcc + kWsPartials + f * (3 + (uint64_t)t->snaps) + l;
 }
 
 // One step from the working state into dst (dst != working state).
@@ -388,11 +410,12 @@ int run_plan(fdb_tape* t, size_t i, bool forward_only, hipStream_t s, const void
 int ensure_partials(fdb_tape* t, int64_t nb) {
   const size_t pb = (size_t)nb * 6 * sizeof(double);
   if (pb > t->partials_bytes) {
-    if (t->partials) TAPE_HIP(hipFree(t->partials));
+    if (t->partials && t->partials_own) TAPE_HIP(hipFree(t->partials));
     t->partials = nullptr;
     t->partials_bytes = 0;
     TAPE_HIP(hipMalloc((void**)&t->partials, pb));
     t->partials_bytes = pb;
+    t->partials_own = true;
   }
   return FDB_OK;
 }
@@ -473,9 +496,12 @@ int fdb_ckpt_plan(int nsteps, int snaps, int* actions, int* args, int cap,
   return (int)std::min<size_t>(p.acts.size(), (size_t)INT32_MAX);
 }
 
-int fdb_tape_create(int ndims, const uint64_t* num_cells, const double* velocity,
-                    const double* lengths, double delta_time, int nsteps, int f_dtype,
-                    int lam_dtype, uint64_t max_bytes, fdb_tape_t** out) {
+namespace {
+
+// The checked arguments as a tape with its schedule and no memory yet.
+int new_tape(int ndims, const uint64_t* num_cells, const double* velocity, const double* lengths,
+             double delta_time, int nsteps, int f_dtype, int lam_dtype, uint64_t max_bytes,
+             fdb_tape_t** out) {
   if (!out) return tfail(FDB_ERR_INVALID, "tape_create: out is null");
   *out = nullptr;
   fdb::Grid3 g;
@@ -509,6 +535,20 @@ int fdb_tape_create(int ndims, const uint64_t* num_cells, const double* velocity
   }
   t->snaps = (int)std::min<uint64_t>((max_bytes - fixed) / t->fbytes, (uint64_t)(nsteps - 1));
   t->plan = make_plan(nsteps, t->snaps);
+  *out = t;
+  return FDB_OK;
+}
+
+}  // namespace
+
+int fdb_tape_create(int ndims, const uint64_t* num_cells, const double* velocity,
+                    const double* lengths, double delta_time, int nsteps, int f_dtype,
+                    int lam_dtype, uint64_t max_bytes, fdb_tape_t** out) {
+  fdb_tape* t = nullptr;
+  if (int rc = new_tape(ndims, num_cells, velocity, lengths, delta_time, nsteps, f_dtype,
+                        lam_dtype, max_bytes, out ? &t : nullptr))
+    return rc;
+  *out = nullptr;
   auto fail_free = [&](hipError_t e, const char* what) {
     (void)hipGetLastError();
     tape_free(t);
@@ -530,17 +570,76 @@ int fdb_tape_create(int ndims, const uint64_t* num_cells, const double* velocity
   return FDB_OK;
 }
 
+int fdb_tape_create_in(int ndims, const uint64_t* num_cells, const double* velocity,
+                       const double* lengths, double delta_time, int nsteps, int f_dtype,
+                       int lam_dtype, uint64_t max_bytes, int method, fdb_tape_t** out,
+                       uint64_t* workspace_bytes) {
+  if (out) *out = nullptr;
+  if (!workspace_bytes) return tfail(FDB_ERR_INVALID, "tape_create_in: workspace_bytes is null");
+  if (method != FDB_GRAD_CHECKPOINT && method != FDB_GRAD_SHIFT)
+    return tfail(FDB_ERR_INVALID, "tape_create_in: unknown method");
+  fdb_tape* t = nullptr;
+  if (int rc = new_tape(ndims, num_cells, velocity, lengths, delta_time, nsteps, f_dtype,
+                        lam_dtype, max_bytes, out ? &t : nullptr))
+    return rc;
+  t->external = true;
+  t->method = method;
+  t->slots.assign(t->snaps, nullptr);
+  *workspace_bytes = ws_bytes(t);
+  *out = t;
+  return FDB_OK;
+}
+
+int fdb_tape_set_workspace(fdb_tape_t* t, void* workspace, uint64_t bytes) {
+  if (!t || !t->external)
+    return tfail(FDB_ERR_INVALID, "tape_set_workspace: not a tape of fdb_tape_create_in");
+  // A checkpointed backward reads the states its forward stored there.
+  if (t->method == FDB_GRAD_CHECKPOINT) t->forward_done = false;
+  t->ws_set = false;
+  if (!workspace) return FDB_OK;
+  if (bytes < ws_bytes(t) || (uintptr_t)workspace % 256 != 0)
+    return tfail(FDB_ERR_INVALID, "tape_set_workspace: workspace too small or not 256-byte "
+                                  "aligned");
+  char* p = (char*)workspace;
+  t->acc = (double*)p;
+  p += kWsAcc;
+  if (!t->partials || !t->partials_own) {  // (a larger buffer of the tape's own stays)
+    t->partials = (double*)p;
+    t->partials_bytes = kWsPartials;
+    t->partials_own = false;
+  }
+  p += kWsPartials;
+  const uint64_t f = ws_align(t->fbytes), l = ws_align(t->lbytes);
+  if (t->method == FDB_GRAD_SHIFT) {
+    t->scratch[0] = p;
+    t->lam_tmp = p;
+  } else {
+    t->base = p;
+    t->scratch[0] = p + f;
+    t->scratch[1] = p + 2 * f;
+    p += 3 * f;
+    t->lam_tmp = p;
+    p += l;
+    for (size_t i = 0; i < t->slots.size(); ++i) t->slots[i] = p + i * f;
+    t->slots_ready = true;
+  }
+  t->ws_set = true;
+  return FDB_OK;
+}
+
 int fdb_tape_forward(fdb_tape_t* t, const void* f0, void* fT, void* stream) {
   if (!t || !f0 || !fT) return tfail(FDB_ERR_INVALID, "tape_forward: null argument");
   if (f0 == fT) return tfail(FDB_ERR_INVALID, "tape_forward: f0 and fT must differ");
+  if (t->external && !t->ws_set) return tfail(FDB_ERR_INVALID, "tape_forward: no workspace set");
   hipStream_t s = (hipStream_t)stream;
   t->fwd_steps = 0;
   t->adj_steps = 0;
   if (t->method == FDB_GRAD_SHIFT) {
-    // Plain forward from the caller's f0 (only read), kept for the products.
-    t->w = f0;
-    t->wstep = 0;
-    if (int rc = advance(t, t->nsteps, fT, s)) return rc;
+    // Plain forward from the caller's f0 (only read), kept for the products;
+    // the passes alternate between fT and one scratch buffer.
+    TAPE_HIP(fdb::launch_planned_steps(t->f_dtype, t->g, f0, fT, t->scratch[0], t->nsteps,
+                                       t->time_block, s, 0, 0));
+    t->fwd_steps = t->nsteps;
     t->f0_ref = f0;
     TAPE_HIP(hipStreamSynchronize(s));
     t->forward_done = true;
@@ -576,6 +675,7 @@ int fdb_tape_backward(fdb_tape_t* t, const void* lam_T, void* lam0, double* grad
     return tfail(FDB_ERR_INVALID, "tape_backward: null argument");
   if (lam_T == lam0) return tfail(FDB_ERR_INVALID, "tape_backward: lam_T and lam0 must differ");
   if (!t->forward_done) return tfail(FDB_ERR_INVALID, "tape_backward: run tape_forward first");
+  if (t->external && !t->ws_set) return tfail(FDB_ERR_INVALID, "tape_backward: no workspace set");
   hipStream_t s = (hipStream_t)stream;
   if (t->method == FDB_GRAD_SHIFT) return backward_shift(t, lam_T, lam0, grad_v, s);
   // Partial-sum scratch of the adjoint kernel, sized for every buffer
@@ -625,9 +725,11 @@ int fdb_tape_set_time_block(fdb_tape_t* t, int k) {
 int fdb_tape_set_method(fdb_tape_t* t, int method) {
   if (!t || (method != FDB_GRAD_CHECKPOINT && method != FDB_GRAD_SHIFT))
     return tfail(FDB_ERR_INVALID, "tape_set_method: unknown method");
+  if (t->external && method != t->method)  // its workspace is sized for one method
+    return tfail(FDB_ERR_INVALID, "tape_set_method: fixed by fdb_tape_create_in");
   if (method != t->method) t->forward_done = false;  // a backward needs this method's forward
   t->method = method;
-  if (method == FDB_GRAD_SHIFT && t->slots_ready) {
+  if (method == FDB_GRAD_SHIFT && t->slots_ready && !t->external) {
     // No snapshots in this method: give their memory back (a later
     // checkpointed forward allocates them again).
     TAPE_HIP(hipDeviceSynchronize());

@@ -159,6 +159,14 @@ int fdb_advect_dev(int ndims, const uint64_t* num_cells, const double* velocity,
                    const double* lengths, double delta_time, int dtype, void* a, void* b,
                    int nsteps, int time_block, void* stream, int* result_in_b);
 
+/* nsteps of advect from src, which is only read, into dst (src copied there
+ * when nsteps <= 0); tmp is scratch of the field's size.  Three distinct
+ * device buffers; the library's own split into passes
+ * (FDB_TIME_BLOCK_AUTO), stochastic rounding as fdb_advect_dev. */
+int fdb_advect_from_dev(int ndims, const uint64_t* num_cells, const double* velocity,
+                        const double* lengths, double delta_time, int dtype, const void* src,
+                        void* dst, void* tmp, int nsteps, void* stream);
+
 /* The pass depths (steps per launch, in launch order) that an advect of
  * nsteps steps with this time_block (0..8, 0 = FDB_TIME_BLOCK_AUTO) makes
  * for this geometry and dtype, as fdb_upwind_advect and fdb_advect_dev
@@ -231,6 +239,20 @@ typedef struct fdb_tape fdb_tape_t;
 int fdb_tape_create(int ndims, const uint64_t* num_cells, const double* velocity,
                     const double* lengths, double delta_time, int nsteps, int f_dtype,
                     int lam_dtype, uint64_t max_bytes, fdb_tape_t** out);
+/* A tape that allocates no device memory: its buffers lie in a workspace
+ * of at least *workspace_bytes, 256-byte aligned, that the caller sets
+ * before forward and before backward (NULL: none).  method (FDB_GRAD_*) is
+ * fixed here.  FDB_GRAD_CHECKPOINT: one workspace from forward to backward
+ * (setting another discards the forward); FDB_GRAD_SHIFT: scratch of one
+ * call, which may be given back in between.  Both calls return with their
+ * work done, so a workspace may be reused or freed at once.  (More partial
+ * sums than a workspace holds, some 20000 blocks, are allocated by the
+ * tape.) */
+int fdb_tape_create_in(int ndims, const uint64_t* num_cells, const double* velocity,
+                       const double* lengths, double delta_time, int nsteps, int f_dtype,
+                       int lam_dtype, uint64_t max_bytes, int method, fdb_tape_t** out,
+                       uint64_t* workspace_bytes);
+int fdb_tape_set_workspace(fdb_tape_t* t, void* workspace, uint64_t bytes);
 int fdb_tape_forward(fdb_tape_t* t, const void* f0, void* fT, void* stream);
 int fdb_tape_backward(fdb_tape_t* t, const void* lam_T, void* lam0, double* grad_v,
                       void* stream);

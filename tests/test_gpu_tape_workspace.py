@@ -1,0 +1,129 @@
+"""Tapes in a caller's workspace and the copy-free forward against the
+allocating forms: the same bits for both methods and every storage type,
+argument errors before anything is launched, inputs left unchanged."""
+from __future__ import annotations
+
+import ctypes as C
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+SHAPE, V, DT = (12, 40, 100), (-0.4, 0.3, -0.25), 2e-3
+
+
+def _bits(t):
+    return t.view({8: torch.int64, 4: torch.int32, 2: torch.int16}[t.element_size()])
+
+
+def _args(T, fd, ld, max_bytes):
+    from fidibench_amd import _lib as L
+    return (3, L.u64s(SHAPE), L.dbls(V), L.dbls((1, 1, 1)), DT, T, fd, ld, max_bytes)
+
+
+@pytest.mark.parametrize("method", ["checkpoint", "shift"])
+@pytest.mark.parametrize("dtype", ["f64", "f32"])
+@pytest.mark.parametrize("T,slots", [(1, 0), (11, 3), (23, 22)])
+def test_workspace_tape_equals_allocating_tape(method, dtype, T, slots):
+    from fidibench_amd import _lib as L, autograd as A
+    fd = L.DTYPES[dtype]
+    tdt = {"f64": torch.float64, "f32": torch.float32}[dtype]
+    g = torch.Generator(device="cuda").manual_seed(T)
+    f0 = torch.rand(SHAPE, generator=g, device="cuda", dtype=tdt)
+    lamT = torch.randn(SHAPE, generator=g, device="cuda", dtype=tdt)
+    keep = f0.clone()
+    budget = (4 + slots) * f0.numel() * f0.element_size()
+    s = torch.cuda.current_stream().cuda_stream
+    lib = L.lib()
+    h, gv = C.c_void_p(), (C.c_double * 3)()
+    L.check(lib.fdb_tape_create(*_args(T, fd, fd, budget), C.byref(h)))
+    L.check(lib.fdb_tape_set_method(h, L.GRAD_METHODS[method]))
+    fT, lam0 = torch.empty_like(f0), torch.empty_like(f0)
+    L.check(lib.fdb_tape_forward(h, f0.data_ptr(), fT.data_ptr(), s))
+    L.check(lib.fdb_tape_backward(h, lamT.data_ptr(), lam0.data_ptr(), gv, s))
+    lib.fdb_tape_destroy(h)
+    tape = A.Tape(SHAPE, V, (1, 1, 1), DT, T, fd, fd, budget, method=method)
+    for _ in range(2):  # again on the same tape
+        fT2, lam2 = torch.full_like(f0, 7), torch.full_like(f0, 7)
+        tape.forward(f0, fT2)
+        got = tape.backward(lamT, lam2)
+        assert torch.equal(_bits(fT2), _bits(fT)) and torch.equal(_bits(lam2), _bits(lam0))
+        assert got == list(gv)
+    assert torch.equal(f0, keep)
+    tape.close()
+
+
+def test_large_checkpointed_tapes_allocate_their_own_states(monkeypatch):
+    from fidibench_amd import _lib as L, autograd as A
+    f0 = torch.rand(SHAPE, device="cuda", dtype=torch.float64)
+    out = []
+    for most in (A._WORKSPACE_MAX, 0):
+        monkeypatch.setattr(A, "_WORKSPACE_MAX", most)
+        tape = A.Tape(SHAPE, V, (1, 1, 1), DT, 9, L.F64, L.F64, 1 << 28)
+        assert (tape._ws is None) == (most == 0)
+        fT, lam0 = torch.empty_like(f0), torch.empty_like(f0)
+        tape.forward(f0, fT)
+        out.append((fT, lam0, tape.backward(f0, lam0)))
+        tape.close()
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
+    assert out[0][2] == out[1][2]
+
+
+def test_workspace_errors():
+    from fidibench_amd import _lib as L
+    lib, s = L.lib(), torch.cuda.current_stream().cuda_stream
+    f = torch.rand(SHAPE, device="cuda", dtype=torch.float64)
+    fT = torch.empty_like(f)
+    h, need = C.c_void_p(), C.c_uint64()
+    a = _args(5, L.F64, L.F64, 1 << 30)
+    assert lib.fdb_tape_create_in(*a, 2, C.byref(h), C.byref(need)) == L.ERR_INVALID
+    assert lib.fdb_tape_create_in(*a, 1, C.byref(h), None) == L.ERR_INVALID
+    few = _args(5, L.F64, L.F64, 1 << 10)
+    assert lib.fdb_tape_create_in(*few, 0, C.byref(h), C.byref(need)) == L.ERR_NOMEM
+    L.check(lib.fdb_tape_create_in(*a, L.GRAD_CHECKPOINT, C.byref(h), C.byref(need)))
+    assert lib.fdb_tape_forward(h, f.data_ptr(), fT.data_ptr(), s) == L.ERR_INVALID
+    ws = torch.empty(need.value + 256, dtype=torch.uint8, device="cuda")
+    assert lib.fdb_tape_set_workspace(h, ws.data_ptr(), need.value - 1) == L.ERR_INVALID
+    assert lib.fdb_tape_set_workspace(h, ws.data_ptr() + 8, need.value) == L.ERR_INVALID
+    assert lib.fdb_tape_set_method(h, L.GRAD_SHIFT) == L.ERR_INVALID
+    L.check(lib.fdb_tape_set_workspace(h, ws.data_ptr(), need.value))
+    L.check(lib.fdb_tape_forward(h, f.data_ptr(), fT.data_ptr(), s))
+    L.check(lib.fdb_tape_set_workspace(h, ws.data_ptr() + 256, need.value))  # drops the forward
+    gv = (C.c_double * 3)()
+    lam0 = torch.empty_like(f)
+    assert lib.fdb_tape_backward(h, f.data_ptr(), lam0.data_ptr(), gv, s) == L.ERR_INVALID
+    lib.fdb_tape_destroy(h)
+
+
+@pytest.mark.parametrize("dtype", ["f64", "f32", "bf16", "bf16sr"])
+@pytest.mark.parametrize("shape", [SHAPE, (30, 70), (41,)])
+@pytest.mark.parametrize("n", [0, 1, 2, 9, 25])
+def test_advect_from_equals_advect(dtype, shape, n):
+    from fidibench_amd import _lib as L
+    nd, code = len(shape), L.DTYPES[dtype]
+    tdt = {"f64": torch.float64, "f32": torch.float32}.get(dtype, torch.bfloat16)
+    f0 = torch.rand(shape, device="cuda").to(tdt)
+    keep, dst, tmp = f0.clone(), torch.empty_like(f0), torch.empty_like(f0)
+    s = torch.cuda.current_stream().cuda_stream
+    geo = (nd, L.u64s(shape), L.dbls(V[:nd]), L.dbls((1,) * nd), DT, code)
+    L.check(L.lib().fdb_advect_from_dev(*geo, f0.data_ptr(), dst.data_ptr(), tmp.data_ptr(), n, s))
+    a, b, r = f0.clone(), torch.empty_like(f0), C.c_int()
+    L.check(L.lib().fdb_advect_dev(*geo, a.data_ptr(), b.data_ptr(), n, 1, s, C.byref(r)))
+    assert torch.equal(_bits(dst), _bits(b if r.value else a))
+    assert torch.equal(_bits(f0), _bits(keep))
+    assert L.lib().fdb_advect_from_dev(*geo, f0.data_ptr(), dst.data_ptr(), dst.data_ptr(), n,
+                                       s) == L.ERR_INVALID
+
+
+def test_forward_without_gradient_keeps_its_input_and_takes_strided_fields():
+    from fidibench_amd import autograd as A
+    big = torch.rand((12, 40, 200), device="cuda", dtype=torch.float64)
+    f0, keep = big[:, :, ::2], big.clone()
+    v = torch.tensor(V, dtype=torch.float64)
+    got = A.advect(f0, v, DT, 13)
+    ref = A.advect(f0.clone().requires_grad_(True), v, DT, 13).detach()
+    assert torch.equal(got, ref) and torch.equal(big, keep)
+    assert torch.equal(A.advect(f0, v, DT, 0), f0)
