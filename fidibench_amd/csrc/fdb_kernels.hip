@@ -1366,10 +1366,12 @@ int64_t resident_blocks(Kern kern, int threads) {
 // (R, WY) pairs the rows kernel is instantiated for (FDB_ROWS_V below).
 constexpr int kRowsShapes[][2] = {{8, 2}, {4, 2}, {4, 4}, {8, 1}, {2, 4}, {2, 8}, {2, 2}, {1, 8}};
 // (R, K, WY) of the temporally blocked forward (FDB_TB below).
-constexpr int kTbShapes[][3] = {{9, 2, 4}, {9, 3, 4}, {9, 4, 4}, {9, 6, 8},
-                                {9, 7, 8}, {9, 8, 8}, {5, 8, 8}};
-// FP64-only shapes: two planes per trip fit in 256 VGPRs.
-constexpr int kTbShapes64[][3] = {{8, 6, 8}, {8, 7, 8}, {7, 8, 8}};
+constexpr int kTbShapes[][3] = {{9, 2, 4}, {9, 3, 4}, {9, 4, 4}, {9, 6, 8}, {9, 7, 8}, {9, 8, 8},
+                                {5, 8, 8}, {2, 2, 8}, {2, 3, 8}, {2, 4, 8}, {8, 6, 8}};
+// FP64-only shapes (7 and 8 rows: two planes per trip fit in 256 VGPRs).
+constexpr int kTbShapes64[][3] = {{8, 7, 8}, {7, 8, 8}, {4, 4, 8}, {4, 6, 8}};
+// FP32- and bf16-only shapes.
+constexpr int kTbShapesLow[][3] = {{6, 4, 8}};
 
 // Default launch shape of the rows kernel.  bytes: storage of the stepped
 // field (lam for the adjoint); fbytes: the adjoint's f_t storage (0: none).
@@ -1440,6 +1442,9 @@ bool tb_shape_ok(const TbCfg& c, int K, int bytes) {
     if (s[0] == c.R && s[1] == K && s[2] == c.WY) return true;
   if (bytes == 8)
     for (const auto& s : kTbShapes64)
+      if (s[0] == c.R && s[1] == K && s[2] == c.WY) return true;
+  if (bytes < 8)
+    for (const auto& s : kTbShapesLow)
       if (s[0] == c.R && s[1] == K && s[2] == c.WY) return true;
   return false;
 }
@@ -1689,6 +1694,113 @@ int fp64_k6_rows(const Grid3& g) {
   return c8 < c9 ? 8 : 9;
 }
 
+// ---- launches over fewer cells than 512^3: a model of the pass's time.
+//
+// A tile's planes follow one another, so such a launch is bound by its
+// longest chain of planes as much as by throughput: fewer rows per wave
+// (shorter planes) and shorter chunks (fewer planes, at the price of K
+// warm-up planes each) both shorten the chain.  A plane of a block takes
+// its waves' vector instructions -- 11 per row and level, `row` per row
+// once -- at the rate of the waves then on a SIMD (a single wave issues
+// every 5 to 6 cycles, four every 4.4), and `sync` per level for the
+// exchange; rounds of resident blocks add up; memory adds in the third
+// power (either bounds the pass).  Constants fitted to 6600 launches on
+// 14 grids of 16^3 to 430 x 420 x 410 cells, every shape and chunk; rms
+// error 8 %, and the shape and chunk picked are within 10 % of the best
+// measured of each depth (16 % where HBM binds, at most 26).
+struct PassModel {
+  double launch;      // us
+  double rate[4];     // ns per instruction and wave, 1..4 waves per SIMD
+  double sync, row;   // us per level; instructions per row and plane
+  double bw;          // MB per us
+};
+constexpr int64_t kModelCells = 1ll << 27;
+const PassModel& pass_model(int bytes) {
+  static constexpr PassModel m64 = {3.66, {1.991, 1.602, 1.409, 1.438}, 0.031, 16.2, 5.37e6};
+  static constexpr PassModel m32 = {4.06, {1.242, 0.809, 0.746, 0.714}, 0.093, 26.1, 5.01e6};
+  static constexpr PassModel m16 = {3.33, {1.284, 0.937, 0.887, 0.773}, 0.103, 31.7, 7.00e6};
+  return bytes == 8 ? m64 : (bytes == 4 ? m32 : m16);
+}
+
+// Shapes to pick from, by depth, with the blocks a CU holds of each (FP64;
+// FP32 and bf16).  Measured at 96^3 FP64, us per launch: K = 4 with 2, 4
+// and 9 rows 9.2, 10.1, 12.2; K = 6 with 4, 8 and 9 rows 15.3, 22.9, 26.1;
+// 256^3: K = 6 with 4 and 8 rows 75.5, 83.4.  (FP32 K = 6 with 4 rows is
+// left out: it is no faster per step than K = 4 with 6.)
+struct PassShape {
+  int K, R, WY, occ64, occ32;
+};
+constexpr PassShape kPassShapes[] = {
+    {2, 2, 8, 4, 4}, {2, 9, 4, 4, 8}, {3, 2, 8, 4, 4}, {3, 9, 4, 3, 6}, {4, 2, 8, 4, 4},
+    {4, 4, 8, 3, 0}, {4, 6, 8, 0, 4}, {4, 9, 4, 3, 5}, {6, 4, 8, 2, 0}, {6, 8, 8, 1, 2},
+    {6, 9, 8, 1, 2}, {7, 8, 8, 1, 0}, {7, 9, 8, 0, 2}, {8, 9, 8, 1, 2}};
+
+struct PassPick {
+  TbCfg cfg{0, 0, 0};
+  int64_t chunk = 0;
+  double us = 0.0;  // 0: no pick
+};
+
+PassPick pick_pass(int bytes, const Grid3& g, int K) {
+  const PassModel& m = pass_model(bytes);
+  PassPick best;
+  const int64_t n0 = g.n[0];
+  const double mem = 2.0 * (double)g.ntot * bytes / m.bw;
+  for (const PassShape& s : kPassShapes) {
+    const int occ = bytes == 8 ? s.occ64 : s.occ32;
+    if (s.K != K || occ == 0 || s.WY * s.R <= K) continue;
+    const int64_t tiles = ((g.n[2] + (64 - K) - 1) / (64 - K)) *
+                          ((g.n[1] + (s.WY * s.R - K) - 1) / (s.WY * s.R - K));
+    auto plane = [&](int64_t blocks_per_cu) {
+      const double w = (double)blocks_per_cu * s.WY / 4.0;  // waves per SIMD
+      const double x = std::min(4.0, std::max(1.0, w)) - 1.0;
+      const int i = std::min(2, (int)x);
+      const double rate = m.rate[i] + (x - i) * (m.rate[i + 1] - m.rate[i]);
+      return w * s.R * (11.0 * K + m.row) * rate * 1e-3 + K * m.sync;
+    };
+    auto consider = [&](int64_t chunk) {
+      const int64_t blocks = tiles * ((n0 + chunk - 1) / chunk);
+      const int64_t cap = (int64_t)occ * 256, full = blocks / cap, rest = blocks - full * cap;
+      double t = (double)full * plane(occ);
+      if (rest) t += plane((rest + 255) / 256);
+      t *= (double)(chunk + K);
+      t = m.launch + std::cbrt(t * t * t + mem * mem * mem);
+      if (best.us == 0.0 || t < best.us) best = PassPick{TbCfg{s.R, s.WY, 0}, chunk, t};
+    };
+    for (int64_t c = 1; c <= std::min<int64_t>(24, n0); ++c) consider(c);
+    for (int64_t nch = 1; nch <= 24; ++nch)
+      if ((n0 + nch - 1) / nch > 24) consider((n0 + nch - 1) / nch);
+  }
+  return best;
+}
+
+// The picks of every depth for the last few (type, grid) pairs.
+struct PassPicks {
+  PassPick k[kMaxTimeBlock + 1];
+};
+PassPicks pass_picks(int bytes, const Grid3& g) {
+  struct Entry {
+    int bytes;
+    int64_t n[3];
+    PassPicks p;
+  };
+  static std::mutex mu;
+  static Entry cache[16];
+  static int used = 0, next = 0;
+  std::lock_guard<std::mutex> lock(mu);
+  for (int i = 0; i < used; ++i) {
+    const Entry& e = cache[i];
+    if (e.bytes == bytes && e.n[0] == g.n[0] && e.n[1] == g.n[1] && e.n[2] == g.n[2]) return e.p;
+  }
+  Entry& e = cache[next];
+  e = Entry{bytes, {g.n[0], g.n[1], g.n[2]}, {}};
+  for (int K = 2; K <= kMaxTimeBlock; ++K)
+    if (!tuning().tb_env[bytes][K]) e.p.k[K] = pick_pass(bytes, g, K);
+  next = (next + 1) % 16;
+  used = std::min(used + 1, 16);
+  return e.p;
+}
+
 // visits != nullptr: launch nothing; store the pass's length in row-plane
 // visits of one resident block slot instead (rounds of resident blocks x
 // planes per block, warm-up planes included, x rows per wave), from the same
@@ -1701,8 +1813,15 @@ hipError_t tb_dispatch(const Grid3& g, const TS* in, TS* out, int K, hipStream_t
   const bool sr = sr_keys != nullptr;
   if (sr && (sizeof(TS) != 2 || !tb_sr_ok(g, K))) return hipErrorNotSupported;
   TbCfg cfg = sr ? tb_sr_cfg(K) : tb_cfg((int)sizeof(TS), K);
-  if constexpr (sizeof(TS) == 8) {
-    if (K == 6 && !sr && levels == nullptr && !tuning().tb_env[8][6]) cfg.R = fp64_k6_rows(g);
+  int64_t chunk = 0;  // 0: from the kernel's occupancy
+  if (!sr && levels == nullptr) {
+    const PassPick pick = g.ntot < kModelCells ? pass_picks((int)sizeof(TS), g).k[K] : PassPick{};
+    if (pick.us > 0.0) {
+      cfg = pick.cfg;
+      chunk = pick.chunk;
+    } else if (sizeof(TS) == 8 && K == 6 && !tuning().tb_env[8][6]) {
+      cfg.R = fp64_k6_rows(g);
+    }
   }
   const int R = cfg.R, WY = cfg.WY;
   if (!(g.act[0] && g.act[1] && g.act[2]) || WY * R <= K) return hipErrorNotSupported;
@@ -1733,12 +1852,14 @@ hipError_t tb_dispatch(const Grid3& g, const TS* in, TS* out, int K, hipStream_t
     auto kern = tb_kernel<TS, RR, KK, W, L1, L2, MD>;                                       \
     const int64_t cap = resident_blocks(kern, 64 * W);                                      \
     int64_t nch;                                                                            \
-    if (cfg.blocks > 0) {                                                                   \
+    if (chunk > 0) {                                                                        \
+      nch = (a.n0 + chunk - 1) / chunk;                                                     \
+    } else if (cfg.blocks > 0) {                                                            \
       nch = std::max<int64_t>(1, (cfg.blocks + tiles / 2) / tiles);                         \
     } else {                                                                                \
       nch = march_chunks(tiles, a.n0, KK, cap, 1, 64, true);                                \
     }                                                                                       \
-    a.chunk = (a.n0 + nch - 1) / nch;                                                       \
+    a.chunk = chunk > 0 ? chunk : (a.n0 + nch - 1) / nch;                                   \
     a.ntiles = tiles * ((a.n0 + a.chunk - 1) / a.chunk);                                    \
     if (visits) {                                                                           \
       *visits = (a.ntiles + cap - 1) / cap * (a.chunk + KK) * RR;                           \
@@ -1759,8 +1880,14 @@ hipError_t tb_dispatch(const Grid3& g, const TS* in, TS* out, int K, hipStream_t
   FDB_TB(9, 7, 8, kTbPlain)
   FDB_TB(9, 8, 8, kTbPlain)
   FDB_TB(5, 8, 8, kTbPlain)
+  FDB_TB(2, 2, 8, kTbPlain)
+  FDB_TB(2, 3, 8, kTbPlain)
+  FDB_TB(2, 4, 8, kTbPlain)
+  FDB_TB(8, 6, 8, kTbPlain)
+  if constexpr (sizeof(TS) == 4 || sizeof(TS) == 2) FDB_TB(6, 4, 8, kTbPlain)
   if constexpr (sizeof(TS) == 8) {
-    FDB_TB(8, 6, 8, kTbPlain)
+    FDB_TB(4, 4, 8, kTbPlain)
+    FDB_TB(4, 6, 8, kTbPlain)
     FDB_TB(8, 7, 8, kTbPlain)
     FDB_TB(7, 8, 8, kTbPlain)
     FDB_TB(9, 4, 4, kTbStoreAll)
@@ -1923,33 +2050,23 @@ bool fused_pass_supported(int dtype, const Grid3& g, int k) {
 }
 
 namespace {
-// Device time (us) of one launch on MI355X, on cubic grids of kPassSide[i]^3
-// cells: index 1 the one-step kernel, 2..8 the fused pass of that many
-// steps (0: no such pass).  Rows: FP64, FP32, bf16 round to nearest, bf16
-// stochastic rounding.  Below 512^3 a launch's time is bound by the
-// latency of its few marched planes rather than by throughput (at 16^3 a
-// one-step FP64 launch, 16 planes in sequence, takes longer than a 4-step
-// pass), so the times are measured points, not a model.
-constexpr int kPassSizes = 4;
-constexpr double kPassSide[kPassSizes] = {16, 128, 256, 512};
-constexpr float kPassUsAt[kPassSizes][4][kMaxTimeBlock + 1] = {
-    {{0, 23.4f, 7.9f, 8.8f, 9.9f, 0, 20.5f, 23.4f, 32.3f},
-     {0, 12.1f, 6.8f, 8.8f, 10.2f, 0, 17.9f, 23.8f, 26.5f},
-     {0, 11.0f, 9.3f, 8.5f, 9.9f, 0, 20.9f, 25.6f, 28.3f},
-     {0, 10.8f, 6.7f, 0, 10.5f, 0, 0, 0, 37.7f}},
-    {{0, 11.2f, 11.3f, 14.7f, 20.5f, 0, 30.2f, 35.2f, 44.4f},
-     {0, 6.0f, 10.5f, 13.0f, 16.2f, 0, 29.0f, 37.5f, 44.8f},
-     {0, 6.1f, 10.8f, 13.2f, 17.6f, 0, 28.0f, 41.1f, 49.5f},
-     {0, 5.9f, 13.5f, 0, 24.8f, 0, 0, 0, 76.4f}},
-    {{0, 62.8f, 65.0f, 66.9f, 67.9f, 0, 88.3f, 100.4f, 114.5f},
-     {0, 30.4f, 39.2f, 41.5f, 43.4f, 0, 57.0f, 70.8f, 80.2f},
-     {0, 17.7f, 28.9f, 35.8f, 44.6f, 0, 72.5f, 78.7f, 91.7f},
-     {0, 20.7f, 33.9f, 0, 67.7f, 0, 0, 0, 144.0f}},
-    {{0, 373, 573, 576, 537, 0, 549, 577, 705},
-     {0, 190, 379, 407, 381, 0, 400, 450, 402},
-     {0, 99, 228, 233, 241, 0, 394, 356, 453},
-     {0, 117, 220, 0, 348, 0, 0, 0, 769}}};
-constexpr const float (&kPassUs)[4][kMaxTimeBlock + 1] = kPassUsAt[kPassSizes - 1];
+// Device time (us) of one launch on MI355X at 512^3: index 1 the one-step
+// kernel, 2..8 the fused pass of that many steps (0: no such pass).  Rows:
+// FP64, FP32, bf16 round to nearest, bf16 stochastic rounding.
+constexpr float kPassUs[4][kMaxTimeBlock + 1] = {
+    {0, 373, 573, 576, 537, 0, 549, 577, 705},
+    {0, 190, 379, 407, 381, 0, 400, 450, 402},
+    {0, 99, 228, 233, 241, 0, 394, 356, 453},
+    {0, 117, 220, 0, 348, 0, 0, 0, 769}};
+// Stochastic rounding on cubic grids of kSrSide[i]^3 cells (its passes
+// pair rows, so their shapes do not follow the grid).
+constexpr int kSrSizes = 4;
+constexpr double kSrSide[kSrSizes] = {16, 128, 256, 512};
+constexpr float kSrUsAt[kSrSizes][kMaxTimeBlock + 1] = {
+    {0, 3.9f, 6.7f, 0, 10.5f, 0, 0, 0, 37.7f},
+    {0, 5.9f, 13.5f, 0, 24.8f, 0, 0, 0, 76.4f},
+    {0, 20.7f, 33.9f, 0, 67.7f, 0, 0, 0, 144.0f},
+    {0, 117, 220, 0, 348, 0, 0, 0, 769}};
 constexpr int kPlanTail = 48;  // steps split exactly; longer runs first take the best depth
 int pass_row(int dtype) {
   return dtype == FDB_F64 ? 0 : (dtype == FDB_F32 ? 1 : (dtype == FDB_BF16 ? 2 : 3));
@@ -1986,10 +2103,8 @@ int64_t fused_pass_visits(int dtype, const Grid3& g, int k) {
 // equal time per plane there, so the length captures rounds of resident
 // blocks, warm-up planes and tiles cut by the grid's extents; at 1024^3 FP64
 // this picks 8-step passes, 679 us per step, over 7-step ones, 710).  On
-// smaller grids launch times stop scaling that way (a march of few planes is
-// bound by the latency of each plane, not by throughput), and each time is
-// interpolated between the measured sizes, linearly in log(time) against
-// log(cells) (grids below 16^3 take the 16^3 times).
+// smaller grids the pass's own model (pick_pass) and, for stochastic
+// rounding, measured times (below 16^3 cells those of 16^3).
 struct PassCosts {
   float us[kMaxTimeBlock + 1];
 };
@@ -2022,15 +2137,30 @@ PassCosts pass_costs(int dtype, const Grid3& g) {
       if (k == 1 || plane_pass_supported(dtype, g, k)) c.us[k] = plane_pass_us(dtype, g, k);
     return c;
   }
+  if (cells < 1.0 && dtype != FDB_BF16_SR) {
+    // One step: a launch, then its fields at the rate of the Infinity Cache
+    // or of HBM (64^3 to 384^3, all types, within 25 %).
+    const double bytes = 2.0 * (double)g.ntot * (double)dtype_size(dtype);
+    c.us[1] = (float)(3.6 + bytes / (bytes <= (double)kResidentBytes ? 6.6e6 : 5.2e6));
+    const PassPicks p = pass_picks((int)dtype_size(dtype), g);
+    for (int k = 2; k <= kMaxTimeBlock; ++k) {
+      if (!fused_pass_supported(dtype, g, k)) continue;
+      c.us[k] = (float)p.k[k].us;
+      if (p.k[k].us <= 0.0 && kPassUs[row][k] > 0.0f)  // a shape set by a tuning variable
+        c.us[k] = (float)(4.0 + kPassUs[row][k] * cells);
+    }
+    return c;
+  }
   if (cells < 1.0) {
-    // Between the measured sizes i and i + 1 (side^3 cells each).
+    // Stochastic rounding: between the measured sizes i and i + 1, linearly
+    // in log(time) against log(cells).
     const double lc = std::log((double)g.ntot);
     int i = 0;
-    while (i + 2 < kPassSizes && lc > 3.0 * std::log(kPassSide[i + 1])) ++i;
-    const double l0 = 3.0 * std::log(kPassSide[i]), l1 = 3.0 * std::log(kPassSide[i + 1]);
+    while (i + 2 < kSrSizes && lc > 3.0 * std::log(kSrSide[i + 1])) ++i;
+    const double l0 = 3.0 * std::log(kSrSide[i]), l1 = 3.0 * std::log(kSrSide[i + 1]);
     const double a = std::min(1.0, std::max(0.0, (lc - l0) / (l1 - l0)));
     for (int k = 1; k <= kMaxTimeBlock; ++k) {
-      const float t0 = kPassUsAt[i][row][k], t1 = kPassUsAt[i + 1][row][k];
+      const float t0 = kSrUsAt[i][k], t1 = kSrUsAt[i + 1][k];
       if (t0 <= 0.0f || t1 <= 0.0f || (k > 1 && !fused_pass_supported(dtype, g, k))) continue;
       c.us[k] = (float)std::exp((1.0 - a) * std::log((double)t0) + a * std::log((double)t1));
     }
