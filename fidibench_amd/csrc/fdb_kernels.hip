@@ -858,7 +858,7 @@ struct TbAux {
 // Raw buffer access to one row: the row's start (uniform) goes into the
 // resource, the lane's byte offset into a VGPR, so no lane does 64-bit
 // address arithmetic.  Offsets stay below the row length (no access is
-// dropped); stores are nontemporal (aux 2).
+// dropped).
 template <typename T>
 __device__ inline __amdgpu_buffer_rsrc_t row_rsrc(const T* row, int bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(row), 0, bytes, 0x00020000);
@@ -873,14 +873,18 @@ __device__ inline float buf_ld(__amdgpu_buffer_rsrc_t rs, uint32_t off, const fl
 __device__ inline uint16_t buf_ld(__amdgpu_buffer_rsrc_t rs, uint32_t off, const uint16_t*) {
   return __builtin_amdgcn_raw_buffer_load_b16(rs, off, 0, 0);
 }
-__device__ inline void buf_st_nt(double v, __amdgpu_buffer_rsrc_t rs, uint32_t off) {
-  __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2_t, v), rs, off, 0, 2);
+// Stores: through the caches, or streaming past them (NT).
+template <bool NT>
+__device__ inline void buf_st(double v, __amdgpu_buffer_rsrc_t rs, uint32_t off) {
+  __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2_t, v), rs, off, 0, NT ? 2 : 0);
 }
-__device__ inline void buf_st_nt(float v, __amdgpu_buffer_rsrc_t rs, uint32_t off) {
-  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rs, off, 0, 2);
+template <bool NT>
+__device__ inline void buf_st(float v, __amdgpu_buffer_rsrc_t rs, uint32_t off) {
+  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rs, off, 0, NT ? 2 : 0);
 }
-__device__ inline void buf_st_nt(uint16_t v, __amdgpu_buffer_rsrc_t rs, uint32_t off) {
-  __builtin_amdgcn_raw_buffer_store_b16(v, rs, off, 0, 2);
+template <bool NT>
+__device__ inline void buf_st(uint16_t v, __amdgpu_buffer_rsrc_t rs, uint32_t off) {
+  __builtin_amdgcn_raw_buffer_store_b16(v, rs, off, 0, NT ? 2 : 0);
 }
 
 // x mod n in [0, n) for any x (n > 0).
@@ -990,6 +994,18 @@ __global__ __launch_bounds__(64 * WY) void tb_kernel(const TS* __restrict__ in,
   constexpr bool kTwoPlanes = !PROD && (K <= 6 || (sizeof(M) == 8 && R * K == 56));
   constexpr bool kCondPrefetch = PIPE && !kTwoPlanes;
   constexpr bool kWaitBeforeStores = (MODE == kTbPlain || MODE == kTbSR) && !kCondPrefetch;
+  // The result's stores.  A tile's rows end inside cache lines that the
+  // neighbouring tile, on the same XCD at about the same time, completes:
+  // through the caches the halves meet in L2, and the next pass finds the
+  // field in the Infinity Cache if it fits.  Measured, streaming / cached,
+  // us a step in passes in turn over two fields: FP32 K = 6, 7, 8 (rows of
+  // 232, 228, 224 bytes per tile) at 512^3 59.6 / 50.4, 61.6 / 52.5, 48.6 /
+  // 49.2, at 768^3 240 / 230, 242 / 214, 155 / 149; bf16 K = 7 at 1024^3
+  // 380 / 352; FP64 4 rows K = 6 at 256^3 14.6 / 13.5.  The FP64 shapes of
+  // large grids lose (K = 7 512^3 91.7 / 93.1, 1024 x 1024 x 768 559 / 605,
+  // K = 8 768^3 270 / 277) and stream, as do the two-row shapes, whose
+  // grids stay in the L2s (96^3 10.4 / 10.6 us a pass).
+  constexpr bool kStream = R == 2 || (sizeof(TS) == 8 && R >= 7 && WY == 8);
   // PROD: fv[l] holds the state of level l at the current plane (LASTP:
   // fv[0], the last level's); after its level it is reloaded with the next
   // plane's (always a valid plane, so every load is unconditional).  The
@@ -1214,7 +1230,7 @@ __global__ __launch_bounds__(64 * WY) void tb_kernel(const TS* __restrict__ in,
           TS* ob = (TS*)adj.lv[l] + pw * plane;
 #pragma unroll
           for (int r = 0; r < R; ++r)
-            if (row_out[r]) buf_st_nt(St<TS>::st(x[r]), row_rsrc(ob + roff[r], rbytes), cb);
+            if (row_out[r]) buf_st<true>(St<TS>::st(x[r]), row_rsrc(ob + roff[r], rbytes), cb);
         }
       }
     }
@@ -1233,7 +1249,7 @@ __global__ __launch_bounds__(64 * WY) void tb_kernel(const TS* __restrict__ in,
       TS* ob = out + pw * plane;
 #pragma unroll
       for (int r = 0; r < R; ++r)
-        if (row_out[r]) buf_st_nt(St<TS>::st(x[r]), row_rsrc(ob + roff[r], rbytes), cb);
+        if (row_out[r]) buf_st<kStream>(St<TS>::st(x[r]), row_rsrc(ob + roff[r], rbytes), cb);
     }
 #pragma unroll
     for (int r = 0; r < R; ++r) x[r] = nx[r];
