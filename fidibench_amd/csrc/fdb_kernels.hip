@@ -96,6 +96,8 @@ __device__ inline uint32_t sr_round(uint32_t x) {
 
 // sr_round(w ^ k) with its first, xor-linear step done on each operand
 // beforehand: sr_round_pre(w ^ (w >> 16) ^ k ^ (k >> 16)) == sr_round(w ^ k).
+// (The product from 16-bit ones, v_dot2_u32_u16 for the cross terms,
+// measured slower than v_mul_lo_u32: 374 against 355 us per 4-step pass.)
 __host__ __device__ inline uint32_t sr_fold(uint32_t x) { return x ^ (x >> 16); }
 __device__ inline uint32_t sr_round_pre(uint32_t x) {
   x *= 0x7feb352du;
@@ -142,6 +144,16 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 __device__ inline uint32_t pack_bf16x2(float lo, float hi) {
   const f32x2 v = {lo, hi};
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+}
+
+// Storage bits of a value that has been through rnd (or the stochastic
+// rounding): for bf16 its high half, no conversion.
+template <typename TS>
+__device__ inline TS st_rounded(typename St<TS>::M x) {
+  if constexpr (sizeof(TS) == 2)
+    return (uint16_t)(__builtin_bit_cast(uint32_t, x) >> 16);
+  else
+    return x;
 }
 
 template <typename TS, int VEC>
@@ -974,16 +986,17 @@ __global__ __launch_bounds__(64 * WY) void tb_kernel(const TS* __restrict__ in,
   for (int l = 0; l < K; ++l)
 #pragma unroll
     for (int r = 0; r < R; ++r) prev[l][r] = M(0);
-  M x[R], nx[R];
+  M x[R];
+  TS nx[R];  // the next plane's rows as stored
   int64_t pw = pmod(first, a.n0);  // wrapped index of the current plane
   {
     const TS* base = in + pw * plane;
 #pragma unroll
-    for (int r = 0; r < R; ++r) x[r] = St<TS>::ld(buf_ld(row_rsrc(base + roff[r], rbytes), cb, in));
+    for (int r = 0; r < R; ++r) nx[r] = buf_ld(row_rsrc(base + roff[r], rbytes), cb, in);
+#pragma unroll
+    for (int r = 0; r < R; ++r) x[r] = St<TS>::ld(nx[r]);  // (nx: defined where a prefetch is skipped)
 #pragma unroll
     for (int r = 0; r < R; ++r) settle(x[r]);
-#pragma unroll
-    for (int r = 0; r < R; ++r) nx[r] = x[r];  // defined where a prefetch is skipped
   }
   // Two planes per trip of the plane loop (the registers of prev[l] and of
   // level l alternate between planes instead of being copied at the end of
@@ -1053,7 +1066,7 @@ __global__ __launch_bounds__(64 * WY) void tb_kernel(const TS* __restrict__ in,
       // K > 6 keeps the branch (unconditional loads there spill).
       const TS* base = in + (m + 1 < cnt ? pn : pw) * plane;
 #pragma unroll
-      for (int r = 0; r < R; ++r) nx[r] = St<TS>::ld(buf_ld(row_rsrc(base + roff[r], rbytes), cb, in));
+      for (int r = 0; r < R; ++r) nx[r] = buf_ld(row_rsrc(base + roff[r], rbytes), cb, in);
     }
     double ps[3] = {0.0, 0.0, 0.0};  // PROD: this plane's products (LASTP: last level)
 #pragma unroll
@@ -1140,7 +1153,7 @@ __global__ __launch_bounds__(64 * WY) void tb_kernel(const TS* __restrict__ in,
         if constexpr (WY > 1) {
           // The next plane's row wr (its level 0) as late as possible, so
           // the plane's prefetch has the whole plane to arrive.
-          if (l + 1 == K) edge[buf ^ 1][w][lane] = nx[wr];
+          if (l + 1 == K) edge[buf ^ 1][w][lane] = St<TS>::ld(nx[wr]);
           lds_barrier();
         }
       } else {
@@ -1154,6 +1167,11 @@ __global__ __launch_bounds__(64 * WY) void tb_kernel(const TS* __restrict__ in,
         d0[r] = prev[l][r] - x[r];
         d2[r] = n2 - x[r];
         if (r != er) d1[r] = x[LO1 ? r - 1 : r + 1] - x[r];
+        // Computed here, in the block of the lane shift, so that the two
+        // become one v_sub_f32_dpp (sunk below the barrier they do not):
+        // bf16 K = 4, 7, 8 at 512^3 237, 351, 449 -> 219, 336, 436 us, FP32
+        // K = 8 390 -> 378 (K = 7 335 -> 341, left out).
+        if constexpr (sizeof(M) == 4 && !PROD && !(sizeof(TS) == 4 && K == 7)) settle(d2[r]);
       }
       M n1 = x[er];  // the block's upwind edge: halo row, any value
       if constexpr (WY > 1) {
@@ -1230,7 +1248,7 @@ __global__ __launch_bounds__(64 * WY) void tb_kernel(const TS* __restrict__ in,
           TS* ob = (TS*)adj.lv[l] + pw * plane;
 #pragma unroll
           for (int r = 0; r < R; ++r)
-            if (row_out[r]) buf_st<true>(St<TS>::st(x[r]), row_rsrc(ob + roff[r], rbytes), cb);
+            if (row_out[r]) buf_st<true>(st_rounded<TS>(x[r]), row_rsrc(ob + roff[r], rbytes), cb);
         }
       }
     }
@@ -1249,10 +1267,10 @@ __global__ __launch_bounds__(64 * WY) void tb_kernel(const TS* __restrict__ in,
       TS* ob = out + pw * plane;
 #pragma unroll
       for (int r = 0; r < R; ++r)
-        if (row_out[r]) buf_st<kStream>(St<TS>::st(x[r]), row_rsrc(ob + roff[r], rbytes), cb);
+        if (row_out[r]) buf_st<kStream>(st_rounded<TS>(x[r]), row_rsrc(ob + roff[r], rbytes), cb);
     }
 #pragma unroll
-    for (int r = 0; r < R; ++r) x[r] = nx[r];
+    for (int r = 0; r < R; ++r) x[r] = St<TS>::ld(nx[r]);
     pw = pn;
   };
   if constexpr (WY > 1 && PIPE) {
@@ -2071,9 +2089,9 @@ namespace {
 // FP64, FP32, bf16 round to nearest, bf16 stochastic rounding.
 constexpr float kPassUs[4][kMaxTimeBlock + 1] = {
     {0, 373, 573, 576, 537, 0, 549, 577, 705},
-    {0, 190, 379, 407, 381, 0, 400, 450, 402},
-    {0, 99, 228, 233, 241, 0, 394, 356, 453},
-    {0, 117, 220, 0, 348, 0, 0, 0, 769}};
+    {0, 190, 331, 333, 333, 0, 344, 381, 378},
+    {0, 99, 163, 172, 220, 0, 402, 347, 440},
+    {0, 115, 167, 0, 325, 0, 0, 0, 729}};
 // Stochastic rounding on cubic grids of kSrSide[i]^3 cells (its passes
 // pair rows, so their shapes do not follow the grid).
 constexpr int kSrSizes = 4;
@@ -2081,8 +2099,8 @@ constexpr double kSrSide[kSrSizes] = {16, 128, 256, 512};
 constexpr float kSrUsAt[kSrSizes][kMaxTimeBlock + 1] = {
     {0, 3.9f, 6.7f, 0, 10.5f, 0, 0, 0, 37.7f},
     {0, 5.9f, 13.5f, 0, 24.8f, 0, 0, 0, 76.4f},
-    {0, 20.7f, 33.9f, 0, 67.7f, 0, 0, 0, 144.0f},
-    {0, 117, 220, 0, 348, 0, 0, 0, 769}};
+    {0, 19.2f, 33.0f, 0, 64.0f, 0, 0, 0, 140.0f},
+    {0, 115, 167, 0, 325, 0, 0, 0, 729}};
 constexpr int kPlanTail = 48;  // steps split exactly; longer runs first take the best depth
 int pass_row(int dtype) {
   return dtype == FDB_F64 ? 0 : (dtype == FDB_F32 ? 1 : (dtype == FDB_BF16 ? 2 : 3));
