@@ -86,7 +86,8 @@ hipError_t launch_fused_pass(int dtype, const Grid3& g, const void* src, void* d
 bool fused_pass_supported(int dtype, const Grid3& g, int k);
 
 // A 2-D problem (axes 1 and 2): its fused passes are plane_kernel's
-// (fdb_plane.hip), of 2..8 steps for FP64, FP32 and bf16 round to nearest.
+// (fdb_plane.hip), of 2..8 steps for FP64, FP32 and bf16 round to nearest,
+// and for FP64 and FP32 its one-step launches too.
 inline bool is_plane(const Grid3& g) { return !g.act[0] && g.act[1] && g.act[2]; }
 bool plane_pass_supported(int dtype, const Grid3& g, int k);
 // hipErrorNotSupported unless plane_pass_supported; src is only read.

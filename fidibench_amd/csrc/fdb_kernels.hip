@@ -2323,7 +2323,11 @@ hipError_t launch_advect_pass(int dtype, const Grid3& g, void* const bufs[2], in
       }
       if (err != hipErrorNotSupported) return err;
     }
-    if (done == 0) {
+    if (done == 0 && plane_pass_supported(dtype, g, 1)) {
+      err = launch_plane_pass(dtype, g, src, dst, 1, s);
+      if (err != hipSuccess) return err;
+      done = 1;
+    } else if (done == 0) {
       switch (dtype) {
         case FDB_F64: err = step_typed<double>(g, src, dst, s); break;
         case FDB_F32: err = step_typed<float>(g, src, dst, s); break;

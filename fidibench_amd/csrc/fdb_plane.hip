@@ -1,5 +1,5 @@
-// fdb_plane.hip -- several upwind steps of a 2-D field in one pass over
-// memory (Upwind<2>, pletzer/fidibench upwind/cxx/upwind.cxx:64-84; the
+// fdb_plane.hip -- one or several upwind steps of a 2-D field in one pass
+// over memory (Upwind<2>, pletzer/fidibench upwind/cxx/upwind.cxx:64-84; the
 // 3-D pass is tb_kernel in fdb_kernels.hip).
 //
 // A wave owns 64 lanes x 2 consecutive columns, H = K rounded up to even of
@@ -15,8 +15,8 @@
 //
 // Bound: vector-ALU issue (6 operations and one 64-bit lane move per two
 // cells and level) where the fields fit the Infinity Cache, HBM beyond it.
-// 2000 x 3000 FP64: 8 steps 21.8 us, 2.7 us a step against 25.1 one step
-// per launch; 8000 x 8000 FP64 (HBM) 25.4 us a step against 205.  Two
+// 2000 x 3000 FP64: 8 steps 21.8 us, 2.7 us a step against 14.6 one step
+// per launch; 8000 x 8000 FP64 (HBM) 25.4 us a step against 180.  Two
 // columns per lane measured 21.8 us against 25.8 with one (more halo and
 // lane moves) and 27.4 with four (fewer waves); a prefetch of two rows 21.8
 // against 24.1 with four (the loop no longer fits well).
@@ -36,7 +36,10 @@ namespace {
 constexpr int kCols = 2;          // columns per lane
 constexpr int kWidth = 64 * kCols;
 constexpr int kWaves = 4;         // independent waves per block
-constexpr int kPrefetch = 2;      // rows loaded ahead
+// Rows loaded ahead.  One step: all rows of a chunk (kStepChunk and the
+// one before it), so a wave has its whole work in flight at once.
+constexpr int prefetch(int k) { return k == 1 ? 4 : 2; }
+constexpr int kStepChunk = prefetch(1) - 1;
 
 using u32x2 = uint32_t __attribute__((ext_vector_type(2)));
 using u32x4 = uint32_t __attribute__((ext_vector_type(4)));
@@ -156,7 +159,7 @@ __global__ __launch_bounds__(64 * kWaves) void plane_kernel(const TS* __restrict
                                                             typename Cell<TS>::M c2) {
   using C = Cell<TS>;
   using M = typename C::M;
-  constexpr int H = K + (K & 1), AUX = NT ? 2 : 0;
+  constexpr int H = K + (K & 1), AUX = NT ? 2 : 0, kPrefetch = prefetch(K);
   constexpr uint32_t kDropped = 0x7ffffff0u;  // past any row's end
   int64_t t = blockIdx.x;
   {  // blocks go to the 8 XCDs in turn: a contiguous range of tiles for each
@@ -255,12 +258,13 @@ constexpr int64_t kWaveSlots = 1024;  // one wave on each SIMD
 // chunks measured best (8000 x 8000: 203 us at 20 rows, 229 at 64).
 int64_t plane_chunk(const Grid3& g, int k, int64_t tiles2) {
   const int64_t n1 = g.n[1];
+  if (k == 1) return std::min<int64_t>(kStepChunk, n1);
   auto waves = [&](int64_t c) { return tiles2 * ((n1 + c - 1) / c); };
   if (waves(20) > 8 * kWaveSlots) return std::min<int64_t>(20, n1);
   int64_t best = n1;
   double least = -1.0;
   for (int64_t c = std::min<int64_t>(4, n1); c <= std::min<int64_t>(n1, 512); ++c) {
-    const int64_t rows = (c + k + kPrefetch - 1) / kPrefetch * kPrefetch;
+    const int64_t rows = (c + k + prefetch(k) - 1) / prefetch(k) * prefetch(k);
     const double per = std::max(1.3, (double)((waves(c) + kWaveSlots - 1) / kWaveSlots));
     if (least < 0.0 || (double)rows * per < least) {
       least = (double)rows * per;
@@ -315,6 +319,9 @@ hipError_t launch_typed(const Grid3& g, const void* src, void* dst, int k, hipSt
   const TS* in = (const TS*)src;
   TS* out = (TS*)dst;
   switch (k) {
+    case 1:
+      if constexpr (sizeof(TS) > 2) return launch_k<TS, 1>(g, in, out, s);
+      return hipErrorNotSupported;
     case 2: return launch_k<TS, 2>(g, in, out, s);
     case 3: return launch_k<TS, 3>(g, in, out, s);
     case 4: return launch_k<TS, 4>(g, in, out, s);
@@ -328,9 +335,13 @@ hipError_t launch_typed(const Grid3& g, const void* src, void* dst, int k, hipSt
 
 }  // namespace
 
+// One step too where it is the faster launch, us by rows_kernel / here:
+// FP64 2000 x 3000 24.7 / 14.6, 703 x 1214 6.5 / 4.0, 8000 x 8000 277 /
+// 180; FP32 10.2 / 9.4, 5.7 / 3.6, 157 / 90; not bf16 (8.4 / 8.9, 56 / 61),
+// whose 16-byte lanes there hold eight cells.
 bool plane_pass_supported(int dtype, const Grid3& g, int k) {
-  if (k < 2 || k > kMaxTimeBlock || !is_plane(g)) return false;
-  if (dtype != FDB_F64 && dtype != FDB_F32 && dtype != FDB_BF16) return false;
+  if (k < 1 || k > kMaxTimeBlock || !is_plane(g)) return false;
+  if (dtype != FDB_F64 && dtype != FDB_F32 && (dtype != FDB_BF16 || k == 1)) return false;
   // 32-bit row offsets, below the one that marks a dropped store.
   return g.n[2] * (int64_t)dtype_size(dtype) < 0x7fffff00LL;
 }
@@ -346,13 +357,16 @@ hipError_t launch_plane_pass(int dtype, const Grid3& g, const void* src, void* d
 }
 
 // Measured on 2000 x 3000 (FP64 17.7, 20.1 and 21.8 us for 4, 6 and 8
-// steps, 25.1 for one; FP32 17.8, bf16 21.2 us for 8), 703 x 1213, 200 x
+// steps, 14.6 for one; FP32 17.8, bf16 21.2 us for 8), 703 x 1213, 200 x
 // 150 and 8000 x 8000: a launch, then the larger of its memory traffic and
 // its waves' time.
 float plane_pass_us(int dtype, const Grid3& g, int k) {
   const double bytes = 2.0 * (double)g.ntot * (double)dtype_size(dtype);
   const bool resident = bytes <= (double)(256ll << 20);
-  if (k == 1) return (float)(3.5 + bytes / (resident ? 4.4e6 : 5.0e6));
+  if (k == 1) {
+    if (dtype != FDB_F64 && dtype != FDB_F32) return (float)(3.5 + bytes / 5.0e6);
+    return (float)(3.0 + bytes / (resident ? 8.3e6 : 5.7e6));
+  }
   const PlaneArgs a = plane_args(g, k);
   const double level = dtype == FDB_F64 ? 0.0285 : (dtype == FDB_F32 ? 0.021 : 0.026);
   const double waves = (double)a.ntiles / (double)kWaveSlots;
