@@ -136,6 +136,7 @@ struct fdb_tape {
   double* partials = nullptr;
   size_t partials_bytes = 0;
   double* acc = nullptr;
+  fdb::PartialSums sums;  // of the backward that runs
   bool forward_done = false;
   bool fuse_adj = false;  // this backward may use fused transpose passes
   int64_t fwd_steps = 0, adj_steps = 0;
@@ -376,8 +377,7 @@ int run_plan(fdb_tape* t, size_t i, bool forward_only, hipStream_t s, const void
           fs[0] = t->w;
           for (int q = 1; q < k; ++q) fs[q] = stack_buffer(t, n - 1 - q);
           const hipError_t e = fdb::launch_adjoint_fused(
-              t->lam_dtype, t->f_dtype, t->g, *lam_next, dst, fs, k, t->partials,
-              (int64_t)(t->partials_bytes / (6 * sizeof(double))), t->acc, s);
+              t->lam_dtype, t->f_dtype, t->g, *lam_next, dst, fs, k, t->sums, s);
           if (e == hipSuccess) {
             for (int q = 1; q < k; ++q) t->stack_steps.pop_back();
             t->w = fs[k - 1];
@@ -393,7 +393,7 @@ int run_plan(fdb_tape* t, size_t i, bool forward_only, hipStream_t s, const void
           if (dst == *lam_next) dst = (dst == lam0) ? t->lam_tmp : lam0;
         }
         TAPE_HIP(fdb::launch_adjoint_step(t->lam_dtype, t->f_dtype, t->g, *lam_next, dst, t->w,
-                                          t->partials, t->acc, s));
+                                          t->sums, s));
         *lam_next = dst;
         ++t->adj_steps;
         break;
@@ -406,10 +406,12 @@ int run_plan(fdb_tape* t, size_t i, bool forward_only, hipStream_t s, const void
   return FDB_OK;
 }
 
-// Grows the adjoint kernel's partial-sum scratch to nb blocks.
+// Grows the adjoint kernel's partial-sum scratch to nb blocks, or to those
+// of every step where they fit in kWsPartials.
 int ensure_partials(fdb_tape* t, int64_t nb) {
-  const size_t pb = (size_t)nb * 6 * sizeof(double);
+  size_t pb = (size_t)nb * 6 * sizeof(double);
   if (pb > t->partials_bytes) {
+    pb = std::max<size_t>(pb, std::min<uint64_t>((uint64_t)pb * t->nsteps, kWsPartials));
     if (t->partials && t->partials_own) TAPE_HIP(hipFree(t->partials));
     t->partials = nullptr;
     t->partials_bytes = 0;
@@ -694,11 +696,13 @@ int fdb_tape_backward(fdb_tape_t* t, const void* lam_T, void* lam0, double* grad
     nb = std::max(nb, fb);
   }
   if (int rc = ensure_partials(t, nb)) return rc;
+  t->sums = {t->partials, (int64_t)(t->partials_bytes / (6 * sizeof(double))), 0, t->acc};
   TAPE_HIP(fdb::launch_zero(t->acc, 6, s));
   const void* lam_next = lam_T;
   int done = 0;
   if (int rc = run_plan(t, t->resume, false, s, &lam_next, lam0, &done, nullptr)) return rc;
   if (done != t->nsteps) return tfail(FDB_ERR_INVALID, "tape_backward: incomplete (internal)");
+  TAPE_HIP(fdb::reduce_partial_sums(t->sums, s));
   if (lam_next != lam0)
     TAPE_HIP(hipMemcpyAsync(lam0, lam_next, t->lbytes, hipMemcpyDeviceToDevice, s));
   double acc[6];
