@@ -251,10 +251,12 @@ __global__ __launch_bounds__(256) void filter_march_kernel(const double* __restr
 // together from the threads' own cells (their queue's middle entry) and
 // the halo ring around them, loaded flat across the block, so every value
 // is read from memory once per plane.  Memory accesses in the plane loop
-// are unconditional, as in the ring kernel.
-template <int R>
+// are unconditional, as in the ring kernel.  Stores go past the caches (NT)
+// only where the fields exceed the Infinity Cache: 256^3 58.3 -> 50.5 us
+// cached, 512^3 416 -> 432.
+template <int R_, int BX, int CX, int CY>
 struct StarShape {
-  static constexpr int kBX = 64, kBY = 4, kCX = 2, kCY = 2;
+  static constexpr int R = R_, kBX = BX, kBY = 256 / BX, kCX = CX, kCY = CY;
   static constexpr int kTX = kBX * kCX, kTY = kBY * kCY;
   static constexpr int kLX = kTX + 2 * R, kLY = kTY + 2 * R, kNE = kLX * kLY;
   static constexpr int kNH = kNE - kTX * kTY;    // halo-ring values per plane
@@ -262,11 +264,11 @@ struct StarShape {
   static constexpr size_t kLds = 2 * (kNE + 64) * sizeof(double);
 };
 
-template <int R>
+template <class S, bool NT>
 __global__ __launch_bounds__(256) void filter_star_kernel(const double* __restrict__ in,
                                                           double* __restrict__ out,
                                                           FilterGeom g, FilterMarch m) {
-  using S = StarShape<R>;
+  constexpr int R = S::R;
   constexpr int BX = S::kBX, BY = S::kBY, CX = S::kCX, CY = S::kCY;
   constexpr int LX = S::kLX, NE = S::kNE, NH = S::kNH, NLH = S::kNLH, D = 2 * R + 1;
   static_assert(R == 1 || R == 2, "the plane loop is unrolled for 4 or 6 queue slots");
@@ -395,7 +397,7 @@ __global__ __launch_bounds__(256) void filter_star_kernel(const double* __restri
 #pragma unroll
         for (int k = 1; k <= R; ++k) acc = acc + g.w[u++] * t[c + k];
         __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, acc), rs, soff[j][i], 0,
-                                              2 /* nt */);
+                                              NT ? 2 : 0);
       }
     }
   };
@@ -420,17 +422,161 @@ __global__ __launch_bounds__(256) void filter_star_kernel(const double* __restri
   }
 }
 
-// Radius R if g is a full 3-D star stencil of radius R = 2 with its terms
-// in map order (see filter_star_kernel), else 0.
-int star_radius(const FilterGeom& g) {
-  for (int R = 2; R <= 2; ++R) {
-    if (g.nt != 6 * R + 1) continue;
+// ---- star block kernel: the star stencils of radius 1 and 2, 3-D or
+// (FLAT) 2-D viewed as n0 x 1 x n1: one block = C planes of a tile, every
+// load of the block issued before the first value is used, one barrier,
+// then all sums.  Fields in the caches are bound by latency and by blocks
+// in flight, not by bytes: a marching block of the kernels around takes its
+// chunk's planes one after the other, each a wait for loads and a barrier,
+// and reads 2R planes before its first output.  Here a block waits once.
+// It reads (C + 2R) / C times the tile instead of about (8 + 2R) / 8,
+// which the L2 and the Infinity Cache serve; from HBM the marching kernels
+// are faster.  us per application, marching (its stores past the caches) ->
+// block: radius 2, 160x144x150 21.9 -> 13.5, 64^3 6.4 -> 4.7, 30x20x19 18.2
+// -> 4.4, 220x220x200 44.8 -> 31.5; radius 1, 160x144x150 21.7 -> 12.1,
+// 256^3 55.8 -> 47.6 (512^3: 395 -> 468, not taken); 2-D radius 1, 64x64
+// 28 -> 4.1, 2000x2048 19.4 -> 11.8, 9000x8000 227 -> 204 (stores past the
+// caches).  32 x 16 tiles: 64 x 8 take 15.9 (radius 2, 160x144x150), 32 x 32
+// 16.9, six planes 14.7, two 21 (32 x 8).
+template <int R_, int BX, int CX, int CY, int C_, bool FLAT_, bool BATCH_>
+struct StarBlock {
+  static constexpr int R = R_, kBX = BX, kBY = 256 / BX, kCX = CX, kCY = CY, C = C_;
+  static constexpr bool FLAT = FLAT_, BATCH = BATCH_;
+  static constexpr int kTX = kBX * kCX, kTY = kBY * kCY;
+  static constexpr int kRY = FLAT ? 0 : R;
+  static constexpr int kLX = kTX + 2 * R, kLY = kTY + 2 * kRY, kNE = kLX * kLY;
+  static constexpr int kNH = kNE - kTX * kTY;          // halo-ring values per plane
+  // ... per thread: of all planes, or of each plane (not BATCH)
+  static constexpr int kNLH = ((BATCH ? C : 1) * kNH + 255) / 256;
+  // LDS plane stride; the spare area for lanes without a ring value is one
+  // of 64 after all planes (BATCH) or after each.
+  static constexpr int kPS = kNE + (BATCH ? 0 : 64);
+  static constexpr int kSpare = BATCH ? C * kNE : kNE;
+  static constexpr int kVals = C * kPS + (BATCH ? 64 : 0);
+};
+
+template <class S, bool NT>
+__global__ __launch_bounds__(256) void filter_star_block_kernel(const double* __restrict__ in,
+                                                                double* __restrict__ out,
+                                                                FilterGeom g, FilterMarch m) {
+  constexpr int R = S::R, C = S::C, BX = S::kBX, BY = S::kBY, CX = S::kCX, CY = S::kCY;
+  constexpr int LX = S::kLX, RY = S::kRY, NH = S::kNH, NLH = S::kNLH;
+  constexpr int PS = S::kPS;
+  __shared__ double tile[S::kVals];
+  const int tx = threadIdx.x, ty = threadIdx.y;
+  const int tid = ty * BX + tx;
+  const int64_t b = xcd_contiguous(blockIdx.x, gridDim.x);
+  const int64_t bx = b % m.tiles_x;
+  const int64_t by = (b / m.tiles_x) % m.tiles_y;
+  const int64_t z0 = b / (m.tiles_x * m.tiles_y) * C;
+  const int64_t x0 = bx * S::kTX, y0 = by * S::kTY;
+  const int64_t plane = g.n[0] * g.n[1];
+
+  int64_t gown[CY][CX];
+  int lown[CY][CX], soff[CY][CX];
+#pragma unroll
+  for (int j = 0; j < CY; ++j)
+#pragma unroll
+    for (int i = 0; i < CX; ++i) {
+      const int64_t x = x0 + tx + BX * i, y = y0 + ty + BY * j;
+      gown[j][i] = filter_wrap(x, 0, g) + g.n[0] * filter_wrap(y, 1, g);
+      lown[j][i] = (ty + BY * j + RY) * LX + tx + BX * i + R;
+      soff[j][i] = (x < g.n[0] && y < g.n[1]) ? (int)((x + g.n[0] * (y - y0)) * 8) : 0x7fffffff;
+    }
+  double q[C + 2 * R][CY][CX];
+#pragma unroll
+  for (int d = 0; d < C + 2 * R; ++d) {
+    const double* pl = in + filter_wrap(z0 - R + d, 2, g) * plane;
+#pragma unroll
+    for (int j = 0; j < CY; ++j)
+#pragma unroll
+      for (int i = 0; i < CX; ++i) q[d][j][i] = pl[gown[j][i]];
+  }
+  // This thread's share of the planes' halo rings: the RY rows above and
+  // below the tile (full width), then R columns left and right of each row.
+  constexpr int NP = S::BATCH ? 1 : C, HP = S::BATCH ? C : 1;  // loads per k, planes per load
+  double h[NLH][NP];
+  int lhal[NLH];
+#pragma unroll
+  for (int k = 0; k < NLH; ++k) {
+    const int e = tid + 256 * k;
+    const int d = e / NH, f = e - d * NH;
+    int lx = 0, ly = 0;
+    if (f < 2 * RY * LX) {
+      ly = f / LX;
+      lx = f - ly * LX;
+      if (ly >= RY) ly += S::kTY;
+    } else {
+      const int f2 = f - 2 * RY * LX;
+      const int row = f2 / (2 * R), c = f2 - row * (2 * R);
+      ly = RY + row;
+      lx = c < R ? c : LX - 2 * R + c;
+    }
+    const bool ok = e < HP * NH;
+    const int64_t at = filter_wrap(x0 - R + lx, 0, g) + g.n[0] * filter_wrap(y0 - RY + ly, 1, g);
+    lhal[k] = ok ? d * PS + ly * LX + lx : S::kSpare + (tid & 63);
+    if constexpr (S::BATCH) {
+      h[k][0] = in[ok ? at + filter_wrap(z0 + d, 2, g) * plane : 0];
+    } else {
+#pragma unroll
+      for (int p = 0; p < NP; ++p) h[k][p] = in[(ok ? at : 0) + filter_wrap(z0 + p, 2, g) * plane];
+    }
+  }
+  const int64_t tile_bytes = (g.n[1] - y0) * g.n[0] * 8;  // tile's first row to the plane's end
+  const int nrec = (int)(tile_bytes < 0x7fffffffLL ? tile_bytes : 0x7fffffffLL);
+#pragma unroll
+  for (int d = 0; d < C; ++d)
+#pragma unroll
+    for (int j = 0; j < CY; ++j)
+#pragma unroll
+      for (int i = 0; i < CX; ++i) tile[d * PS + lown[j][i]] = q[d + R][j][i];
+#pragma unroll
+  for (int k = 0; k < NLH; ++k)
+#pragma unroll
+    for (int p = 0; p < NP; ++p) tile[lhal[k] + p * PS] = h[k][p];
+  lds_barrier();
+#pragma unroll
+  for (int d = 0; d < C; ++d) {
+    if (z0 + d >= g.n[2]) break;  // block-uniform
+    const double* t = tile + d * PS;
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+        out + (z0 + d) * plane + y0 * g.n[0], 0, nrec, 0x00020000);
+#pragma unroll
+    for (int j = 0; j < CY; ++j)
+#pragma unroll
+      for (int i = 0; i < CX; ++i) {
+        const int c = lown[j][i];
+        double acc = 0.0;
+        int u = 0;  // term index in map order
+#pragma unroll
+        for (int k = -R; k < 0; ++k) acc = acc + g.w[u++] * t[c + k];
+#pragma unroll
+        for (int k = -RY; k < 0; ++k) acc = acc + g.w[u++] * t[c + k * LX];
+#pragma unroll
+        for (int k = -R; k <= R; ++k) acc = acc + g.w[u++] * q[d + R + k][j][i];
+#pragma unroll
+        for (int k = 1; k <= RY; ++k) acc = acc + g.w[u++] * t[c + k * LX];
+#pragma unroll
+        for (int k = 1; k <= R; ++k) acc = acc + g.w[u++] * t[c + k];
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, acc), rs, soff[j][i], 0,
+                                              NT ? 2 : 0);
+      }
+  }
+}
+
+// Radius R if g is a full star stencil of radius R = 1 or 2 on axes 0, 2
+// and, unless flat, 1, with its terms in map order (see
+// filter_star_kernel), else 0.
+int star_radius(const FilterGeom& g, bool flat) {
+  for (int R = 1; R <= 2; ++R) {
+    const int ry = flat ? 0 : R;
+    if (g.nt != 4 * R + 2 * ry + 1) continue;
     int expect[kFilterMaxTerms][3] = {};
     int u = 0;
     for (int k = -R; k < 0; ++k) expect[u++][0] = k;
-    for (int k = -R; k < 0; ++k) expect[u++][1] = k;
+    for (int k = -ry; k < 0; ++k) expect[u++][1] = k;
     for (int k = -R; k <= R; ++k) expect[u++][2] = k;
-    for (int k = 1; k <= R; ++k) expect[u++][1] = k;
+    for (int k = 1; k <= ry; ++k) expect[u++][1] = k;
     for (int k = 1; k <= R; ++k) expect[u++][0] = k;
     bool same = true;
     for (int t = 0; t < g.nt && same; ++t)
@@ -440,9 +586,91 @@ int star_radius(const FilterGeom& g) {
   return 0;
 }
 
+// Input and output below this stay in the Infinity Cache from one
+// application to the next (stores go through the caches).
+constexpr int64_t kFilterResident = 256ll << 20;
+// Radius 2 in 3-D: above this the block form's re-read planes cost more than
+// its waits save (148 MiB: 31.5 us against 33.0 marching with cached stores;
+// 185 MiB: 40.2 against 38.0).
+constexpr int64_t kStarBlockMax2 = 160ll << 20;
+
+// Grids with fewer blocks than this (one per CU) take the smaller ones: 64^3
+// radius 2 (128 blocks) 5.7 -> 4.7 us, 101x99x97 (700) 8.4 -> 10.3.
+constexpr int64_t kSmallStarBlocks = 256;
+
+// Calls f(S{}, kernel) for the block form of radius R (FLAT: 2-D).  small:
+// fewer planes per block, for grids with less than a block per CU.
+template <class F>
+hipError_t with_star_block(int R, bool flat, bool small, bool stream, F f) {
+#define FDB_SB(R, BX, CY, C, FL, BA)                                          \
+  do {                                                                        \
+    using S = StarBlock<R, BX, 1, CY, C, FL, BA>;                             \
+    return stream ? f(S{}, &filter_star_block_kernel<S, true>)                \
+                  : f(S{}, &filter_star_block_kernel<S, false>);              \
+  } while (0)
+  if (flat) {
+    if (R == 1 && small) FDB_SB(1, 256, 1, 4, true, true);
+    if (R == 1) FDB_SB(1, 256, 1, 8, true, true);
+    if (small) FDB_SB(2, 256, 1, 4, true, true);
+    FDB_SB(2, 256, 1, 8, true, true);
+  }
+  if (R == 1 && small) FDB_SB(1, 32, 1, 2, false, true);
+  if (R == 1) FDB_SB(1, 32, 2, 4, false, false);
+  if (small) FDB_SB(2, 32, 1, 2, false, true);
+  FDB_SB(2, 32, 2, 4, false, false);
+#undef FDB_SB
+}
+
+template <class S>
+int64_t star_block_tiles(const FilterGeom& g, FilterMarch& m) {
+  m = FilterMarch{};
+  m.rx = m.rz = S::R;
+  m.ry = S::kRY;
+  m.LX = S::kLX;
+  m.LY = S::kLY;
+  m.D = 2 * S::R + 1;
+  m.chunk = S::C;
+  m.tiles_x = (g.n[0] + S::kTX - 1) / S::kTX;
+  m.tiles_y = (g.n[1] + S::kTY - 1) / S::kTY;
+  return m.tiles_x * m.tiles_y * ((g.n[2] + S::C - 1) / S::C);
+}
+
+// The block form's plan for the star stencil g of radius R, or false where a
+// marching kernel measured faster or the grid doesn't fit it.  Any extents
+// do: every coordinate goes through the full wrap.
+bool star_block_plan(const FilterGeom& g, int R, bool flat, FilterPlan* p) {
+  const int64_t bytes = 16 * g.n[0] * g.n[1] * g.n[2];
+  if (!flat && bytes > (R == 1 ? kFilterResident : kStarBlockMax2)) return false;
+  if (16 * g.n[0] * 8 >= 0x7fffffffLL) return false;  // store offsets within a tile
+  p->stream = bytes > kFilterResident;
+  for (bool small : {false, true}) {
+    (void)with_star_block(R, flat, small, p->stream, [&](auto shape, auto) {
+      p->blocks = star_block_tiles<decltype(shape)>(g, p->m);
+      return hipSuccess;
+    });
+    p->block = small ? 2 : 1;
+    if (p->blocks >= kSmallStarBlocks) break;
+  }
+  p->g = g;
+  p->lds = 0;  // static
+  if (p->blocks > 0 && p->blocks <= 0x7fffffffLL) return true;
+  *p = FilterPlan{};
+  return false;
+}
+
+hipError_t launch_star_block(const FilterPlan& p, const double* in, double* out, hipStream_t s) {
+  return with_star_block(p.m.rz, p.kind == kFilterRows, p.block == 2, p.stream,
+                         [&](auto shape, auto kern) {
+                           using S = decltype(shape);
+                           hipLaunchKernelGGL(kern, dim3((unsigned)p.blocks),
+                                              dim3(S::kBX, S::kBY), 0, s, in, out, p.g, p.m);
+                           return hipGetLastError();
+                         });
+}
+
 template <int R>
 bool star_plan(const FilterGeom& g, FilterMarch& m, int64_t& blocks) {
-  using S = StarShape<R>;
+  using S = StarShape<R, 64, 2, 2>;
   m = FilterMarch{};
   m.rx = m.ry = m.rz = R;
   m.LX = S::kLX;
@@ -455,7 +683,7 @@ bool star_plan(const FilterGeom& g, FilterMarch& m, int64_t& blocks) {
   m.tiles_y = (g.n[1] + S::kTY - 1) / S::kTY;
   const int64_t tiles = m.tiles_x * m.tiles_y;
   const int64_t cap =
-      kernel_capacity(reinterpret_cast<const void*>(&filter_star_kernel<R>), 256, 0);
+      kernel_capacity(reinterpret_cast<const void*>(&filter_star_kernel<StarShape<R, 64, 2, 2>, true>), 256, 0);
   const int64_t per_round = std::max<int64_t>(1, cap / tiles);
   const int64_t nch = march_chunks(tiles, g.n[2], 2 * R, cap,
                                    std::max<int64_t>(1, per_round / 2), 4 * per_round, true);
@@ -577,10 +805,12 @@ __global__ __launch_bounds__(kFilterThreads) void filter_sin_kernel(double* __re
 }  // namespace
 
 hipError_t plan_filter(const FilterGeom& g, FilterPlan* p) {
-  // 2-D grids (no axis-2 extent or offsets): rows marched along axis 1,
-  // the grid viewed as n0 x 1 x n1 (same memory order).  3-D grids with
-  // n1 >= 8: full star stencils of radius 2 by the star kernel, others by
-  // planes marched along axis 2 (rings up to 160 KB of LDS).
+  // 2-D grids (no axis-2 extent or offsets): star stencils by the block
+  // kernel, others by rows marched along axis 1, the grid viewed as n0 x 1 x
+  // n1 (same memory order).  3-D grids with n1 >= 8: star stencils by the
+  // block kernel while the fields fit the Infinity Cache, beyond it those of
+  // radius 2 by the star kernel; others by planes marched along axis 2
+  // (rings up to 160 KB of LDS).
   // Otherwise (1-D grids, stencils wider than the ring allows): the
   // gather kernel.
   *p = FilterPlan{};
@@ -598,17 +828,27 @@ hipError_t plan_filter(const FilterGeom& g, FilterPlan* p) {
       h.neg[1][k] = 0;
       h.neg[2][k] = g.neg[1][k];
     }
+    const int star = star_radius(h, true);
+    if (star && star_block_plan(h, star, true, p)) {
+      p->kind = kFilterRows;
+      return hipSuccess;
+    }
     if (march_plan<March2D>(h, p->m, p->lds, p->blocks)) {
       p->kind = kFilterRows;
       p->g = h;
       return hipSuccess;
     }
   }
-  const int star = g.n[2] > 1 ? star_radius(g) : 0;
+  const int star = g.n[2] > 1 ? star_radius(g, false) : 0;
+  if (star && g.n[1] >= March3D::kTY && g.n[2] > 2 * star && star_block_plan(g, star, false, p)) {
+    p->kind = star == 2 ? kFilterStar : kFilterPlanes;
+    return hipSuccess;
+  }
   if (star == 2 && star_plan<2>(g, p->m, p->blocks)) {
     p->kind = kFilterStar;
     p->g = g;
     p->lds = 0;  // static
+    p->stream = 16 * g.n[0] * g.n[1] * g.n[2] > kFilterResident;
     return hipSuccess;
   }
   if (g.n[1] >= March3D::kTY && march_plan<March3D>(g, p->m, p->lds, p->blocks)) {
@@ -636,13 +876,16 @@ hipError_t plan_filter(const FilterGeom& g, FilterPlan* p) {
 }
 
 hipError_t launch_filter(const FilterPlan& p, const double* in, double* out, hipStream_t s) {
+  if (p.block) return launch_star_block(p, in, out, s);
   if (p.kind == kFilterRows) return launch_march<March2D>(p, in, out, s);
   if (p.kind == kFilterPlanes) return launch_march<March3D>(p, in, out, s);
   if (p.kind == kFilterPlanesMid) return launch_march<March3DMid>(p, in, out, s);
   if (p.kind == kFilterPlanesWide) return launch_march<March3DWide>(p, in, out, s);
   if (p.kind == kFilterStar) {
     const dim3 grid((unsigned)p.blocks), block(64, 4);
-    hipLaunchKernelGGL(filter_star_kernel<2>, grid, block, 0, s, in, out, p.g, p.m);
+    auto* kern = p.stream ? &filter_star_kernel<StarShape<2, 64, 2, 2>, true>
+                          : &filter_star_kernel<StarShape<2, 64, 2, 2>, false>;
+    hipLaunchKernelGGL(kern, grid, block, 0, s, in, out, p.g, p.m);
     return hipGetLastError();
   }
   const FilterGeom& g = p.g;

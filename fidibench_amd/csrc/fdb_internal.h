@@ -194,8 +194,11 @@ struct FilterPlan {
   FilterMarch m;
   size_t lds;    // dynamic LDS bytes per block
   int64_t blocks;
+  int block;     // 1, 2: the star block kernel (2: its small blocks); 0: as kind says
+  bool stream;   // star kernels: stores past the caches
 };
 constexpr int kFilterGather = 0;  // one thread per output cell, neighbours from HBM/L2
+// (with FilterPlan::block the star block kernel runs instead of the one named)
 constexpr int kFilterPlanes = 1;  // 3-D: 128 x 8 tiles marched along axis 2
 constexpr int kFilterRows = 2;    // 2-D: 512-wide tiles marched along axis 1
 constexpr int kFilterPlanesWide = 3;  // 3-D, halo tiles up to radius 8
