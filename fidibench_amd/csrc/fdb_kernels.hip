@@ -1790,6 +1790,32 @@ struct PassPick {
   double us = 0.0;  // 0: no pick
 };
 
+// Calls f(chunk) for the candidate planes per tile of n0 planes.
+template <class F>
+void for_chunks(int64_t n0, F f) {
+  for (int64_t c = 1; c <= std::min<int64_t>(24, n0); ++c) f(c);
+  for (int64_t nch = 1; nch <= 24; ++nch)
+    if ((n0 + nch - 1) / nch > 24) f((n0 + nch - 1) / nch);
+}
+
+// The model's time of a pass's arithmetic, us, without its launch: rounds
+// of occ blocks per CU, the last one at what it fills.
+double pass_compute(const PassModel& m, int R, int WY, int K, int64_t tiles, int64_t n0,
+                    int64_t chunk, int64_t occ) {
+  auto plane = [&](int64_t blocks_per_cu) {
+    const double w = (double)blocks_per_cu * WY / 4.0;  // waves per SIMD
+    const double x = std::min(4.0, std::max(1.0, w)) - 1.0;
+    const int i = std::min(2, (int)x);
+    const double rate = m.rate[i] + (x - i) * (m.rate[i + 1] - m.rate[i]);
+    return w * R * (11.0 * K + m.row) * rate * 1e-3 + K * m.sync;
+  };
+  const int64_t blocks = tiles * ((n0 + chunk - 1) / chunk);
+  const int64_t cap = occ * 256, full = blocks / cap, rest = blocks - full * cap;
+  double t = (double)full * plane(occ);
+  if (rest) t += plane((rest + 255) / 256);
+  return t * (double)(chunk + K);
+}
+
 PassPick pick_pass(int bytes, const Grid3& g, int K) {
   const PassModel& m = pass_model(bytes);
   PassPick best;
@@ -1800,26 +1826,30 @@ PassPick pick_pass(int bytes, const Grid3& g, int K) {
     if (s.K != K || occ == 0 || s.WY * s.R <= K) continue;
     const int64_t tiles = ((g.n[2] + (64 - K) - 1) / (64 - K)) *
                           ((g.n[1] + (s.WY * s.R - K) - 1) / (s.WY * s.R - K));
-    auto plane = [&](int64_t blocks_per_cu) {
-      const double w = (double)blocks_per_cu * s.WY / 4.0;  // waves per SIMD
-      const double x = std::min(4.0, std::max(1.0, w)) - 1.0;
-      const int i = std::min(2, (int)x);
-      const double rate = m.rate[i] + (x - i) * (m.rate[i + 1] - m.rate[i]);
-      return w * s.R * (11.0 * K + m.row) * rate * 1e-3 + K * m.sync;
-    };
-    auto consider = [&](int64_t chunk) {
-      const int64_t blocks = tiles * ((n0 + chunk - 1) / chunk);
-      const int64_t cap = (int64_t)occ * 256, full = blocks / cap, rest = blocks - full * cap;
-      double t = (double)full * plane(occ);
-      if (rest) t += plane((rest + 255) / 256);
-      t *= (double)(chunk + K);
+    for_chunks(n0, [&](int64_t chunk) {
+      double t = pass_compute(m, s.R, s.WY, K, tiles, n0, chunk, occ);
       t = m.launch + std::cbrt(t * t * t + mem * mem * mem);
       if (best.us == 0.0 || t < best.us) best = PassPick{TbCfg{s.R, s.WY, 0}, chunk, t};
-    };
-    for (int64_t c = 1; c <= std::min<int64_t>(24, n0); ++c) consider(c);
-    for (int64_t nch = 1; nch <= 24; ++nch)
-      if ((n0 + nch - 1) / nch > 24) consider((n0 + nch - 1) / nch);
+    });
   }
+  return best;
+}
+
+// Planes per tile of a transpose pass of this shape by the same model
+// (march_chunks takes a CU with one of two blocks for half as fast, where
+// two waves per SIMD issue nine tenths of what four do).  By march_chunks
+// and by this, us: FP32 96^3 4 steps 32.3, 23.8, last 8 steps 49.1, 35.4;
+// 120x161x192 last 60.0, 53.2; the same choice elsewhere or within 5 %.
+int64_t adj_chunk(int bytes, int R, int WY, int K, int64_t tiles, int64_t n0, int64_t occ) {
+  int64_t best = n0;
+  double least = -1.0;
+  for_chunks(n0, [&](int64_t chunk) {
+    const double t = pass_compute(pass_model(bytes), R, WY, K, tiles, n0, chunk, occ);
+    if (least < 0.0 || t < least) {
+      least = t;
+      best = chunk;
+    }
+  });
   return best;
 }
 
@@ -1954,11 +1984,14 @@ hipError_t tb_dispatch(const Grid3& g, const TS* in, TS* out, int K, hipStream_t
 }
 
 // Fused transpose pass (tb_kernel with PROD): K adjoint steps with the
-// velocity products, K = 4, 8 waves of 4 rows (FP64) or 8 rows (FP32):
-// prev, the K states and the level's differences then stay within 256
-// VGPRs without spills (FP64 spills from 5 rows on).  LAST: the products
-// of the last step only, against fs[0] (kTbAdjLast): K = 7 with 8 rows
-// (FP64, 234 VGPRs, one block per CU like the plain 7-step pass) or K = 8
+// velocity products, K = 4, 8 waves of 4 rows: prev, the K states and the
+// level's differences then stay within 256 VGPRs without spills (FP64 spills
+// from 5 rows on), and FP32 has two blocks per CU.  FP32 with 8, 6, 5, 4, 3
+// rows (8 and 6 and 5: one block per CU), us per pass at the best chunk: 96^3
+// 33.6, 29.9, 26.7, 23.8, 22.0; 120x161x192 51.2, 45.7, 46.1, 45.0, 47.7;
+// 256^3 163, 145, 157, 141, 151; 512^3 929, 899, 932, 876, 889.  LAST: the
+// products of the last step only, against fs[0] (kTbAdjLast): K = 7 with 8
+// rows (FP64, 234 VGPRs, one block per CU like the plain 7-step pass) or K = 8
 // with 6 rows (FP32, at most 115 VGPRs, so two blocks per CU).  *nb_out
 // gets the block count (= partial slots written); with dry = true nothing
 // is launched.  hipErrorNotSupported when the shape has no fused form or
@@ -1969,7 +2002,7 @@ hipError_t tb_adj_dispatch(const Grid3& g, const TS* in, TS* out, const void* co
                            hipStream_t s) {
   using M = typename St<TS>::M;
   if (sizeof(TS) < 4 || K > kMaxTimeBlock) return hipErrorNotSupported;
-  constexpr int R = LAST ? (sizeof(TS) == 8 ? 8 : 6) : (sizeof(TS) == 8 ? 4 : 8), WY = 8;
+  constexpr int R = LAST ? (sizeof(TS) == 8 ? 8 : 6) : 4, WY = 8;
   constexpr int KL = LAST ? (sizeof(TS) == 8 ? 7 : 8) : 4;  // the instantiated depth
   constexpr int MD = LAST ? kTbAdjLast : kTbAdjoint;
   if (!(g.act[0] && g.act[1] && g.act[2]) || WY * R <= K) return hipErrorNotSupported;
@@ -1992,9 +2025,8 @@ hipError_t tb_adj_dispatch(const Grid3& g, const TS* in, TS* out, const void* co
 #define FDB_TBA_DIR(KK, L1, L2)                                                              \
   if (!launched && K == KK && lo1 == L1 && lo2 == L2) {                                      \
     auto kern = tb_kernel<TS, R, KK, WY, L1, L2, MD, TF>;                                    \
-    const int64_t nch =                                                                      \
-        march_chunks(tiles, a.n0, KK, resident_blocks(kern, 64 * WY), 1, 64, true);          \
-    a.chunk = (a.n0 + nch - 1) / nch;                                                        \
+    const int64_t occ = std::max<int64_t>(1, resident_blocks(kern, 64 * WY) / device_cus()); \
+    a.chunk = adj_chunk((int)sizeof(TS), R, WY, KK, tiles, a.n0, occ);                       \
     a.ntiles = tiles * ((a.n0 + a.chunk - 1) / a.chunk);                                     \
     if (nb_out) *nb_out = a.ntiles;                                                          \
     if (dry) return hipSuccess;                                                              \
