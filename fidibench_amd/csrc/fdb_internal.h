@@ -125,6 +125,11 @@ hipError_t launch_planned_steps(int dtype, const Grid3& g, const void* src, void
 // The storage layout of a dtype (FDB_BF16_SR is stored as FDB_BF16).
 inline int storage_dtype(int dtype) { return dtype == 3 ? 2 : dtype; }
 
+// Steps of the next launch_fused_pass with levels (every state kept) in a run
+// of `run` steps, at most `cap` a pass; 0: one-step launches are as fast, or
+// there is no such pass.
+int store_all_steps(int dtype, const Grid3& g, int run, int cap);
+
 // K transpose steps in one pass (lam/f_t storage FP64/FP64, FP32/FP32 or
 // FP32/bf16; all three axes present): lam = (A^T)^K lam_next, where fs[l]
 // is the forward state of the l-th step (f_{t-l} for a pass starting from

@@ -1835,8 +1835,8 @@ PassPick pick_pass(int bytes, const Grid3& g, int K) {
   return best;
 }
 
-// Planes per tile of a transpose pass of this shape by the same model
-// (march_chunks takes a CU with one of two blocks for half as fast, where
+// Planes per tile of a transpose or store-all pass of this shape by the same
+// model (march_chunks takes a CU with one of two blocks for half as fast, where
 // two waves per SIMD issue nine tenths of what four do).  By march_chunks
 // and by this, us: FP32 96^3 4 steps 32.3, 23.8, last 8 steps 49.1, 35.4;
 // 120x161x192 last 60.0, 53.2; the same choice elsewhere or within 5 %.
@@ -1880,6 +1880,21 @@ PassPicks pass_picks(int bytes, const Grid3& g) {
   return e.p;
 }
 
+// Store-all passes (every level written) of the smaller grids: 4 steps by 8
+// waves of 6 rows (FP32) or 4 rows (FP64), in one round of at most a block
+// per CU: with more blocks the five fields' written lines spread over more
+// planes than the caches hold (FP32 256^3: 69 us a pass at one block per CU,
+// 96 to 102 with the chunks of two to four).  us per step, FP32 one-step
+// launches -> this: 96^3 5.0 -> 3.7, 120x161x192 7.4 -> 6.0, 192x200x210
+// 13.4 -> 9.7, 256^3 21.9 -> 17.3, 330x320x310 59 -> 35 (512^3 189 -> 204 to
+// 223); FP64 8 steps by 9 rows -> this: 96^3 6.2 -> 3.7, 120x161x192 9.6 ->
+// 7.6, 192x200x210 19.0 -> 14.2, 240x230x220 25.4 -> 21.4 (256^3 27.2 -> 30.9).
+constexpr int64_t kStoreAllCells32 = 64ll << 20, kStoreAllCells64 = 14ll << 20;
+bool small_store_all(int bytes, const Grid3& g, int K) {
+  return K == 4 && bytes >= 4 && !tuning().tb_env[bytes][K] &&
+         g.ntot < (bytes == 8 ? kStoreAllCells64 : kStoreAllCells32);
+}
+
 // visits != nullptr: launch nothing; store the pass's length in row-plane
 // visits of one resident block slot instead (rounds of resident blocks x
 // planes per block, warm-up planes included, x rows per wave), from the same
@@ -1902,6 +1917,9 @@ hipError_t tb_dispatch(const Grid3& g, const TS* in, TS* out, int K, hipStream_t
       cfg.R = fp64_k6_rows(g);
     }
   }
+  const bool small_all = levels != nullptr && small_store_all((int)sizeof(TS), g, K);
+  if (small_all) cfg = sizeof(TS) == 8 ? TbCfg{4, 8, 0} : TbCfg{6, 8, 0};
+  if (levels != nullptr && sizeof(TS) == 4 && !small_all) return hipErrorNotSupported;
   const int R = cfg.R, WY = cfg.WY;
   if (!(g.act[0] && g.act[1] && g.act[2]) || WY * R <= K) return hipErrorNotSupported;
   TbArgs a;
@@ -1919,8 +1937,9 @@ hipError_t tb_dispatch(const Grid3& g, const TS* in, TS* out, int K, hipStream_t
   Coef<M> cf;
   for (int j = 0; j < 3; ++j) cf.c[j] = (M)g.c[j];
   TbAux aux{};
+  if (small_all) chunk = adj_chunk((int)sizeof(TS), R, WY, K, tiles, a.n0, 1);
   const bool all = levels != nullptr;
-  if (all && sizeof(TS) != 8) return hipErrorNotSupported;
+  if (all && sizeof(TS) < 4) return hipErrorNotSupported;
   for (int l = 0; all && l + 1 < K; ++l) aux.lv[l] = levels[l];
   for (int l = 0; sr && l < K; ++l) a.sr_key[l] = sr_fold(sr_keys[l]);
   const int mode = all ? kTbStoreAll : (sr ? kTbSR : kTbPlain);
@@ -1971,7 +1990,9 @@ hipError_t tb_dispatch(const Grid3& g, const TS* in, TS* out, int K, hipStream_t
     FDB_TB(7, 8, 8, kTbPlain)
     FDB_TB(9, 4, 4, kTbStoreAll)
     FDB_TB(9, 8, 8, kTbStoreAll)
+    FDB_TB(4, 4, 8, kTbStoreAll)
   }
+  if constexpr (sizeof(TS) == 4) FDB_TB(6, 4, 8, kTbStoreAll)
   if constexpr (sizeof(TS) == 2) {
     FDB_TB(8, 2, 4, kTbSR)
     FDB_TB(8, 4, 4, kTbSR)
@@ -2525,6 +2546,14 @@ int64_t adjoint_fused_blocks(int lam_dtype, int f_dtype, const Grid3& g, int k) 
   (void)adj_fused_typed<false>(lam_dtype, f_dtype, g, nullptr, nullptr, nullptr, k, nullptr, 0,
                                &nb, true, nullptr);
   return nb;
+}
+
+int store_all_steps(int dtype, const Grid3& g, int run, int cap) {
+  const int bytes = storage_dtype(dtype) == FDB_F64 ? 8 : (dtype == FDB_F32 ? 4 : 0);
+  const int most = std::min(run, cap);
+  if (bytes == 0 || most < 4) return 0;
+  if (bytes == 4) return small_store_all(4, g, 4) ? 4 : 0;
+  return most >= 8 && !small_store_all(8, g, 4) ? 8 : 4;
 }
 
 int64_t adjoint_blocks(int lam_dtype, int f_dtype, const Grid3& g, const void* lam_next,

@@ -306,8 +306,8 @@ int run_plan(fdb_tape* t, size_t i, bool forward_only, hipStream_t s, const void
           while (i + 2 * run + 1 < acts.size() && acts[i + 2 * run].first == FDB_CK_ADVANCE &&
                  acts[i + 2 * run].second == 1 && acts[i + 2 * run + 1].first == FDB_CK_STORE)
             ++run;
-          const int k = (run >= 8 && t->time_block >= 8) ? 8
-                        : (run >= 4 && t->time_block >= 4) ? 4 : 0;
+          const int k = fdb::store_all_steps(t->f_dtype, t->g, (int)std::min<size_t>(run, 8),
+                                             t->time_block);
           const size_t n = t->stack_steps.size();
           if (k > 0 && n - 1 + (size_t)k <= t->slots.size()) {
             void* lv[fdb::kMaxTimeBlock];
