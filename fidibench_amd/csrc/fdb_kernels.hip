@@ -2277,12 +2277,14 @@ PassCosts pass_costs(int dtype, const Grid3& g) {
   for (int k = 2; k <= kMaxTimeBlock; ++k) {
     if (tab[k] <= 0.0f || ref[k] <= 0 || !fused_pass_supported(dtype, g, k)) continue;
     const int64_t v = fused_pass_visits(dtype, g, k);
-    // No pass is faster than HBM lets the two-step one be, which is bound by
-    // it: its time follows the cells, not the visits (stochastic rounding,
-    // 2 steps: 167 us at 512^3, 291 at 600x620x640, 420 at 768x700x640, 1484 at
-    // 1024^3; by visits alone 1122 at 1024^3, and 2-step passes were picked
-    // there: 742 us a step against 514 in 4-step ones).
-    if (v > 0) c.us[k] = std::max(tab[k] * (float)v / (float)ref[k], tab[2] * (float)cells);
+    if (v > 0) c.us[k] = tab[k] * (float)v / (float)ref[k];
+    // The two-step pass is bound by HBM: its time follows the cells where the
+    // visits grow less (stochastic rounding, 167 us at 512^3, 291 at
+    // 600x620x640, 420 at 768x700x640, 1484 at 1024^3; by visits alone 1122 at
+    // 1024^3, and 2-step passes were picked there: 742 us a step against 514 in
+    // 4-step ones).  Not a bound on deeper passes, whose shapes store better
+    // (FP64 600x900x1000: 6 steps in 2118 us, 2 steps by cells 2305).
+    if (k == 2) c.us[k] = std::max(c.us[k], tab[k] * (float)cells);
   }
   return c;
 }
