@@ -406,7 +406,7 @@ def laplacian(iters=10, with_cpu=True):
                               "traffic": pmc_traffic(name,
                                                      "filter_march_kernel_laplacian_stats.md"),
                               "kernel": {"star": "filter_star_kernel (3-D star stencil)",
-                                         "rows": "filter_march_kernel (rows, 2-D)"}.get(
+                                         "rows": "filter_star_block_kernel (2-D star stencil)"}.get(
                                              flt.kernel(),
                                              f"filter_march_kernel ({flt.kernel()}, 3-D)"),
                               "avg_launch_ms": launch_ms},

@@ -3,9 +3,10 @@
 //
 // The handle mirrors the reference's Upwind<NDIMS> object
 // (pletzer/fidibench upwind/cxx/upwind.cxx:19-135): the field lives in
-// HBM as two ping-pong buffers; checksum()/std()/print()/saveVTK() copy it
-// back in chunks and reproduce the reference's host arithmetic and output
-// byte for byte.
+// HBM as two ping-pong buffers; checksum() and std() fold it on the device in
+// the reference's order and bits (fdb_fold.hip; small fields on the host), and
+// print()/saveVTK() copy it back in chunks and reproduce the reference's
+// output byte for byte.
 #include <hip/hip_runtime_api.h>
 
 #include <algorithm>

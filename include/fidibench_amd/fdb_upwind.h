@@ -80,8 +80,9 @@ int fdb_upwind_destroy(fdb_upwind_t* h);
 int fdb_upwind_advect(fdb_upwind_t* h, int num_time_steps, double delta_time);
 
 /* checksum() const, upwind.cxx:91-93: the sequential left fold from 0.0
- * of the field (widened to double), computed on the host after a copy
- * back, so FP64 results match the reference bit for bit. */
+ * of the field (widened to double): on the device by an exact parallel
+ * form of that fold (fields of 65536 values or more), else on the host;
+ * FP64 results match the reference bit for bit either way. */
 int fdb_upwind_checksum(fdb_upwind_t* h, double* out);
 
 /* std() const, upwind.cxx:95-103. */
