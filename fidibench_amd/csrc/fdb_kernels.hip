@@ -2155,14 +2155,15 @@ namespace {
 // Device time (us) of one launch on MI355X at 512^3: index 1 the one-step
 // kernel, 2..8 the fused pass of that many steps (0: no such pass).  Rows:
 // FP64, FP32, bf16 round to nearest, bf16 stochastic rounding.  bf16's 4, 7
-// and 8 are the geometric mean over 512^3 and six grids to 1024^3 of the time
-// per 512^3-equivalent visits (at 512^3 220, 347, 440), where 4 and 8 steps are
-// within a few percent of each other: by the 512^3 times alone 1024x1024x768
-// ran in 4-step passes, 306 us a step against 254 in 8-step ones.
+// and 8 steps are within a few percent of each other per step at 512^3 (220,
+// 347, 440 us a launch), so their entries come from 24 grids of 512^3 to 1024^3
+// cells: those within the spread of time per visits (7, 4 and 4 %) that pick a
+// depth 1.3 % above the best measured on average (2.9 % by the 512^3 times,
+// which run 1024x1024x768 in 4-step passes, 306 us a step against 256).
 constexpr float kPassUs[4][kMaxTimeBlock + 1] = {
     {0, 373, 573, 576, 537, 0, 549, 577, 705},
     {0, 190, 331, 333, 333, 0, 344, 381, 378},
-    {0, 99, 163, 172, 213, 0, 402, 326, 414},
+    {0, 99, 163, 172, 217, 0, 402, 320, 416},
     {0, 115, 167, 0, 325, 0, 0, 0, 729}};
 // Stochastic rounding on cubic grids of kSrSide[i]^3 cells (its passes
 // pair rows, so their shapes do not follow the grid).
