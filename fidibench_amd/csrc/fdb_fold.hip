@@ -32,6 +32,7 @@
 #include <cstring>
 
 #include "../../include/fidibench_amd/fdb_upwind.h"
+#include "fdb_fold_map.h"
 #include "fdb_internal.h"
 
 #pragma clang fp contract(off)
@@ -66,27 +67,6 @@ struct FoldTerm {
     return d * d;
   }
 };
-
-// Effect of a run of values on m: d[p] is added to an m of parity p; lo
-// and hi bound the offsets from the starting m after each value (both
-// parities; the trajectories of the two differ by at most 1).
-struct FoldMap {
-  double d0, d1, lo, hi;
-};
-
-__device__ inline bool odd(double d) {  // |d| < 2^53, an integer
-  const double h = 0.5 * d;
-  return h != floor(h);
-}
-
-__device__ inline FoldMap then(const FoldMap& a, const FoldMap& b) {
-  FoldMap r;
-  r.d0 = a.d0 + (odd(a.d0) ? b.d1 : b.d0);
-  r.d1 = a.d1 + (odd(a.d1) ? b.d0 : b.d1);  // start 1: parity 1 + d1
-  r.lo = fmin(a.lo, fmin(a.d0, a.d1) + b.lo);
-  r.hi = fmax(a.hi, fmax(a.d0, a.d1) + b.hi);
-  return r;
-}
 
 template <typename TS>
 __global__ __launch_bounds__(kFoldThreads) void fold_sum_kernel(const TS* __restrict__ x,
@@ -164,8 +144,7 @@ __global__ __launch_bounds__(kFoldThreads) void fold_map_kernel(
     any_bad = 0;
     any_value = 0;
   }
-  const FoldMap id = {0.0, 0.0, __builtin_inf(), -__builtin_inf()};
-  FoldMap run = id;  // of the chunk's tiles so far (thread 0)
+  FoldMap run = fold_identity();  // of the chunk's tiles so far (thread 0)
   bool value = false;
   for (uint64_t tb = b; tb < e; tb += kFoldTile) {
 #pragma unroll
@@ -177,35 +156,23 @@ __global__ __launch_bounds__(kFoldThreads) void fold_map_kernel(
       vals[j + j / kFoldPer] = neg ? -v : v;
     }
     __syncthreads();
-    FoldMap m = id;
-    double a0 = 0.0, a1 = 0.0;
+    FoldMap m = fold_identity();
 #pragma unroll
     for (int k = 0; k < kFoldPer; ++k) {
       const double v = ldexp(vals[t * (kFoldPer + 1) + k], scale);
       bad |= !(fabs(v) < kTwo52);
-      const double f = floor(v), r = v - f;
-      double d0 = r > 0.5 ? f + 1.0 : f, d1 = d0;
-      if (r == 0.5) {  // to the even m
-        d0 = odd(a0 + f) ? f + 1.0 : f;
-        d1 = odd(a1 + f) ? f : f + 1.0;
-      }
-      a0 += d0;
-      a1 += d1;
-      m.lo = fmin(m.lo, fmin(a0, a1));
-      m.hi = fmax(m.hi, fmax(a0, a1));
+      fold_append(m, v);
     }
-    m.d0 = a0;
-    m.d1 = a1;
     // Ordered reduction over the wave, then over the waves.
     for (int w = 1; w < 64; w <<= 1) {
       const FoldMap o = {__shfl_down(m.d0, w), __shfl_down(m.d1, w), __shfl_down(m.lo, w),
                          __shfl_down(m.hi, w)};
-      m = then(m, o);  // (lanes that are no multiple of 2w hold leftovers)
+      m = fold_then(m, o);  // (lanes that are no multiple of 2w hold leftovers)
     }
     if ((t & 63) == 0) wave_map[t >> 6] = m;
     __syncthreads();
     if (t == 0)
-      for (int w = 0; w < kFoldThreads / 64; ++w) run = then(run, wave_map[w]);
+      for (int w = 0; w < kFoldThreads / 64; ++w) run = fold_then(run, wave_map[w]);
   }
   if (bad) any_bad = 1;
   if (value) any_value = 1;

@@ -4,7 +4,8 @@
 // instrumented, run by tests/test_host_sanitize.py; never shipped).
 //
 // It calls every entry point whose work is host logic -- the checkpoint
-// schedule, the reference's checksum/std folds, the two VTK writers, the
+// schedule, the reference's checksum/std folds, the maps of the device's
+// parallel form of them, the two VTK writers, the
 // raw-file header checks on good, truncated, foreign and malformed files,
 // the CLI parser, argument validation of the handle/tape/filter
 // constructors (which stop before any device work) and the tuning-variable
@@ -13,6 +14,8 @@
 //
 //   san_host            the checks above
 //   san_host tuning     the same process with malformed tuning variables set
+#include <algorithm>
+#include <cmath>
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
@@ -23,6 +26,8 @@
 #include "../../include/fidibench_amd/CmdLineArgs.hpp"
 #include "../../include/fidibench_amd/fdb_filter.h"
 #include "../../include/fidibench_amd/fdb_upwind.h"
+#include "fdb_fold_map.h"
+#include "fdb_internal.h"
 
 namespace {
 
@@ -84,6 +89,55 @@ void folds_and_vtk() {
         "write_vtk 3d");
   check(fdb_host_write_vtk(1, n1, xmin, len, g.data(), "f", tmp("f.vtk").c_str()) == FDB_OK,
         "write_vtk 1d");
+}
+
+// One value at a time and in runs of 8, 64 and 512 joined pairwise, as the
+// fold kernel's lanes, waves and blocks join them; then the host's step.
+// Values: multiples of a quarter unit and both neighbours of each (ties and
+// what lies next to a tie on either side), of both signs, added to even and
+// odd significands of both signs in several binades.
+void fold_maps() {
+  uint64_t r = 88172645463325252ull;
+  auto rnd = [&] { return r ^= r << 13, r ^= r >> 7, r ^= r << 17; };
+  auto value = [&](double u) {
+    double q = (double)(int64_t)(rnd() % 17) - 8.0;
+    q *= 0.25 * u;
+    const uint64_t side = rnd() % 3;
+    return side == 0 ? q : std::nextafter(q, side == 1 ? -1e300 : 1e300);
+  };
+  int bad = 0;
+  for (int ex : {-900, -3, 0, 1, 52, 53, 700})
+    for (int neg = 0; neg < 2; ++neg)
+      for (int rep = 0; rep < 400; ++rep) {
+        const double u = std::ldexp(1.0, ex - 52);
+        const int n = rep < 200 ? 1 : 512;
+        std::vector<double> x(n);
+        for (double& v : x) v = value(u);
+        const uint64_t m = (3ull << 51) + rnd() % 4;
+        const double s0 = (neg ? -1.0 : 1.0) * std::ldexp((double)m, ex - 52);
+        double want = s0;
+        for (double v : x) want = want + v;
+        std::vector<fdb::FoldMap> runs;
+        for (int i = 0; i < n; i += 8) {
+          fdb::FoldMap f = fdb::fold_identity();
+          for (int k = i; k < std::min(n, i + 8); ++k)
+            fdb::fold_append(f, std::ldexp(neg ? -x[k] : x[k], 52 - ex));
+          runs.push_back(f);
+        }
+        while (runs.size() > 1) {
+          for (size_t i = 0; 2 * i < runs.size(); ++i)
+            runs[i] = fdb::fold_then(runs[2 * i], runs[2 * i + 1]);
+          runs.resize(runs.size() / 2);
+        }
+        const fdb::FoldMap& f = runs[0];
+        double got = s0;
+        const fdb::FoldRec rec{f.d0, f.d1, f.lo, f.hi, ex, neg, fdb::kFoldMapped, -1};
+        const bool applies = fdb::fold_step(rec, nullptr, (uint64_t)n, (uint64_t)n, &got);
+        if ((!applies || got != want) && ++bad <= 4)
+          std::fprintf(stderr, "fold map: n %d ex %d s0 %a x0 %a want %a got %a\n", n, ex, s0, x[0],
+                       want, got);
+      }
+  check(bad == 0, "fold maps equal the sequential loop");
 }
 
 void write_file(const std::string& path, const std::vector<unsigned char>& bytes) {
@@ -218,6 +272,7 @@ int main(int argc, char** argv) {
   } else {
     plans();
     folds_and_vtk();
+    fold_maps();
     raw_headers();
     cli();
     constructors();

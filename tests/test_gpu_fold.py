@@ -86,3 +86,38 @@ def test_filter_checksums(oracle):
     assert flt.computeCheckSum("input") == oracle.checksum(
         np.ascontiguousarray(f.ravel(order="F")))
     flt.close()
+
+
+# The sum of f[:at] is an odd multiple of u, and f[at] (in a chunk of its own
+# from the sum's) lies next to half of u: the loop leaves the sum, a tie would
+# move it to the even neighbour.
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+@pytest.mark.parametrize("low", [1, 2])  # odd and even significands
+@pytest.mark.parametrize("at", [2048, 5000, 65535])
+def test_values_next_to_a_tie(oracle, sign, low, at):
+    from fidibench_amd import Filter, Upwind
+    half = 2.0 ** -53
+    near = [half, np.nextafter(half, 0.0), np.nextafter(half, 1.0),
+            3 * half, np.nextafter(3 * half, 0.0), np.nextafter(3 * half, 1.0)]
+    for v in near + [-x for x in near]:
+        f = np.zeros(65536)
+        f[0], f[at] = sign * (1.5 + low * 2.0 ** -52), sign * v
+        with Upwind((1.0,), (1.0,), (f.size,)) as up:
+            up.set_field(f)
+            assert up.checksum().hex() == oracle.checksum(f).hex(), (sign, low, at, v.hex())
+            assert up.std().hex() == oracle.std(f).hex(), (sign, low, at, v.hex())
+    flt = Filter((256, 256), [0.0, 0.0], [1.0, 1.0], {(0, 0): 1.0})
+    flt.setInData(f)
+    assert flt.computeCheckSum("input").hex() == oracle.checksum(f).hex()
+    flt.close()
+
+
+def test_values_next_to_a_tie_add_up(oracle):
+    from fidibench_amd import Upwind
+    f = np.zeros(65536)
+    f[0] = 1.5 + 2.0 ** -52
+    f[2048:4096:2], f[2049:4096:2] = -np.nextafter(2.0 ** -53, 0.0), 2.0 ** -52
+    for g in (f, -f):
+        with Upwind((1.0,), (1.0,), (g.size,)) as up:
+            up.set_field(g)
+            assert up.checksum().hex() == oracle.checksum(g).hex()
