@@ -37,8 +37,9 @@ def _stream() -> int:
 
 
 # A checkpointed tape whose states take more than this allocates them itself
-# and gives them back to the device when it closes; smaller ones lie in
-# torch memory, whose cache keeps them for the next tape.
+# and gives them back to the device when it closes; smaller ones, and the one
+# scratch field of "shift", lie in torch memory, whose cache keeps them for
+# the next tape.
 _WORKSPACE_MAX = 4 << 30
 
 
@@ -53,7 +54,7 @@ class Tape:
         self.f_dtype, self.lam_dtype = f_dtype, lam_dtype
         self.method = method
         self._f0 = None
-        self._ws = None  # "checkpoint": the states' torch memory
+        self._ws = None  # the working memory, where it is torch's
         h, need = C.c_void_p(), C.c_uint64()
         if method == "shift":
             # No snapshots in this method: ask for the fixed working set only
@@ -67,47 +68,29 @@ class Tape:
                 int(nsteps), f_dtype, lam_dtype, int(max_bytes))
         L.check(L.lib().fdb_tape_create_in(*args, L.GRAD_METHODS[method], C.byref(h),
                                            C.byref(need)))
-        self._h, self._need = h, need.value
-        if method == "checkpoint":
-            if self._need > _WORKSPACE_MAX:
-                self.close()
-                h, self._need = C.c_void_p(), 0
-                L.check(L.lib().fdb_tape_create(*args, C.byref(h)))
-                self._h = h
-            else:
-                self._ws = self._workspace()
-                self._set_workspace(self._ws)
-
-    def _workspace(self) -> torch.Tensor:
+        self._h = h
+        if method == "checkpoint" and need.value > _WORKSPACE_MAX:
+            self.close()
+            h = C.c_void_p()
+            L.check(L.lib().fdb_tape_create(*args, C.byref(h)))
+            self._h = h
+            return
+        # Held until close(): forward and backward allocate nothing.
         try:
-            return torch.empty(self._need, dtype=torch.uint8, device="cuda")
+            self._ws = torch.empty(need.value, dtype=torch.uint8, device="cuda")
         except torch.cuda.OutOfMemoryError as e:
             raise L.FdbError(L.ERR_NOMEM, str(e)) from None
-
-    def _set_workspace(self, ws) -> None:
-        L.check(L.lib().fdb_tape_set_workspace(self._h, None if ws is None else ws.data_ptr(),
-                                               self._need))
-
-    def _call(self, fn, *args) -> None:
-        """fn(tape, *args) on the current stream; "shift" tapes hold scratch
-        for this call only (it returns with its work done)."""
-        if self.method == "shift":
-            ws = self._workspace()
-            self._set_workspace(ws)
-        try:
-            L.check(fn(self._h, *args, _stream()))
-        finally:
-            if self.method == "shift":
-                self._set_workspace(None)
+        L.check(L.lib().fdb_tape_set_workspace(h, self._ws.data_ptr(), need.value))
 
     def forward(self, f0: torch.Tensor, fT: torch.Tensor) -> None:
-        self._call(L.lib().fdb_tape_forward, f0.data_ptr(), fT.data_ptr())
+        L.check(L.lib().fdb_tape_forward(self._h, f0.data_ptr(), fT.data_ptr(), _stream()))
         # "shift" reads f0 again in backward: keep the tensor alive until then.
         self._f0 = f0 if self.method == "shift" else None
 
     def backward(self, lamT: torch.Tensor, lam0: torch.Tensor) -> list:
         gv = (C.c_double * 3)()
-        self._call(L.lib().fdb_tape_backward, lamT.data_ptr(), lam0.data_ptr(), gv)
+        L.check(L.lib().fdb_tape_backward(self._h, lamT.data_ptr(), lam0.data_ptr(), gv,
+                                          _stream()))
         return [gv[i] for i in range(self.ndims)]
 
     def set_time_block(self, k: int) -> None:

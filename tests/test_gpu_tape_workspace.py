@@ -127,3 +127,21 @@ def test_forward_without_gradient_keeps_its_input_and_takes_strided_fields():
     ref = A.advect(f0.clone().requires_grad_(True), v, DT, 13).detach()
     assert torch.equal(got, ref) and torch.equal(big, keep)
     assert torch.equal(A.advect(f0, v, DT, 0), f0)
+
+
+@pytest.mark.parametrize("method", ["checkpoint", "shift"])
+def test_a_tape_allocates_when_it_is_made_only(method):
+    from fidibench_amd import _lib as L, autograd as A
+    f0 = torch.rand(SHAPE, device="cuda", dtype=torch.float64)
+    fT, lam0 = torch.empty_like(f0), torch.empty_like(f0)
+
+    def allocations():
+        return torch.cuda.memory_stats()["allocation.all.allocated"]
+
+    before = allocations()
+    tape = A.Tape(SHAPE, V, (1, 1, 1), DT, 9, L.F64, L.F64, 1 << 28, method=method)
+    made = allocations()
+    tape.forward(f0, fT)
+    tape.backward(f0, lam0)
+    assert made == before + 1 and allocations() == made
+    tape.close()
