@@ -75,22 +75,35 @@ class Tape:
             L.check(L.lib().fdb_tape_create(*args, C.byref(h)))
             self._h = h
             return
-        # Held until close(): forward and backward allocate nothing.
+        # Held until close(): forward and backward allocate nothing.  The memory
+        # is the current stream's; calls on another one wait for what that
+        # stream had queued on the memory's last owner.
+        self._ws_stream = torch.cuda.current_stream()
         try:
             self._ws = torch.empty(need.value, dtype=torch.uint8, device="cuda")
         except torch.cuda.OutOfMemoryError as e:
             raise L.FdbError(L.ERR_NOMEM, str(e)) from None
         L.check(L.lib().fdb_tape_set_workspace(h, self._ws.data_ptr(), need.value))
 
+    def _call_stream(self) -> int:
+        """The current stream, ordered after the work queued on the working
+        memory's own.  (Both calls return with their work done, so nothing
+        else has to wait for them.)"""
+        s = torch.cuda.current_stream()
+        if self._ws is not None and s != self._ws_stream:
+            s.wait_stream(self._ws_stream)
+        return s.cuda_stream
+
     def forward(self, f0: torch.Tensor, fT: torch.Tensor) -> None:
-        L.check(L.lib().fdb_tape_forward(self._h, f0.data_ptr(), fT.data_ptr(), _stream()))
+        L.check(L.lib().fdb_tape_forward(self._h, f0.data_ptr(), fT.data_ptr(),
+                                         self._call_stream()))
         # "shift" reads f0 again in backward: keep the tensor alive until then.
         self._f0 = f0 if self.method == "shift" else None
 
     def backward(self, lamT: torch.Tensor, lam0: torch.Tensor) -> list:
         gv = (C.c_double * 3)()
         L.check(L.lib().fdb_tape_backward(self._h, lamT.data_ptr(), lam0.data_ptr(), gv,
-                                          _stream()))
+                                          self._call_stream()))
         return [gv[i] for i in range(self.ndims)]
 
     def set_time_block(self, k: int) -> None:

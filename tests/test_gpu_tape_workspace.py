@@ -145,3 +145,41 @@ def test_a_tape_allocates_when_it_is_made_only(method):
     tape.backward(f0, lam0)
     assert made == before + 1 and allocations() == made
     tape.close()
+
+
+@pytest.mark.parametrize("method", ["checkpoint", "shift"])
+def test_a_tape_waits_for_the_last_owner_of_its_memory(method):
+    """The tape takes memory that its stream still has work queued on, and is
+    called on another stream."""
+    from fidibench_amd import _lib as L, autograd as A
+    shape, T = (64, 96, 128), 9
+    f0 = torch.rand(shape, device="cuda", dtype=torch.float64)
+    other = torch.cuda.Stream()
+
+    def grad(busy):
+        fT, lam0 = torch.empty_like(f0), torch.empty_like(f0)
+        torch.cuda.synchronize()
+        if busy:
+            old = torch.empty(_need(shape, T, method), dtype=torch.uint8, device="cuda")
+            for i in range(300):
+                old.fill_(i % 251)
+            del old
+        tape = A.Tape(shape, V, (1, 1, 1), DT, T, L.F64, L.F64, 1 << 28, method=method)
+        with torch.cuda.stream(other):
+            tape.forward(f0, fT)
+            gv = tape.backward(f0, lam0)
+        tape.close()
+        return fT, lam0, gv
+
+    a, b = grad(False), grad(True)
+    assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1]) and a[2] == b[2]
+
+
+def _need(shape, T, method):
+    from fidibench_amd import _lib as L
+    h, need = C.c_void_p(), C.c_uint64()
+    L.check(L.lib().fdb_tape_create_in(3, L.u64s(shape), L.dbls(V), L.dbls((1, 1, 1)), DT, T, L.F64,
+                                       L.F64, 1 << 28, L.GRAD_METHODS[method], C.byref(h),
+                                       C.byref(need)))
+    L.lib().fdb_tape_destroy(h)
+    return need.value
