@@ -629,11 +629,11 @@ int fdb_tape_set_workspace(fdb_tape_t* t, void* workspace, uint64_t bytes) {
   return FDB_OK;
 }
 
-int fdb_tape_forward(fdb_tape_t* t, const void* f0, void* fT, void* stream) {
-  if (!t || !f0 || !fT) return tfail(FDB_ERR_INVALID, "tape_forward: null argument");
-  if (f0 == fT) return tfail(FDB_ERR_INVALID, "tape_forward: f0 and fT must differ");
-  if (t->external && !t->ws_set) return tfail(FDB_ERR_INVALID, "tape_forward: no workspace set");
-  hipStream_t s = (hipStream_t)stream;
+}  // extern "C"
+
+namespace {
+
+int forward_run(fdb_tape* t, const void* f0, void* fT, hipStream_t s) {
   t->fwd_steps = 0;
   t->adj_steps = 0;
   if (t->method == FDB_GRAD_SHIFT) {
@@ -671,14 +671,7 @@ int fdb_tape_forward(fdb_tape_t* t, const void* f0, void* fT, void* stream) {
   return FDB_OK;
 }
 
-int fdb_tape_backward(fdb_tape_t* t, const void* lam_T, void* lam0, double* grad_v,
-                      void* stream) {
-  if (!t || !lam_T || !lam0 || !grad_v)
-    return tfail(FDB_ERR_INVALID, "tape_backward: null argument");
-  if (lam_T == lam0) return tfail(FDB_ERR_INVALID, "tape_backward: lam_T and lam0 must differ");
-  if (!t->forward_done) return tfail(FDB_ERR_INVALID, "tape_backward: run tape_forward first");
-  if (t->external && !t->ws_set) return tfail(FDB_ERR_INVALID, "tape_backward: no workspace set");
-  hipStream_t s = (hipStream_t)stream;
+int backward_run(fdb_tape* t, const void* lam_T, void* lam0, double* grad_v, hipStream_t s) {
   if (t->method == FDB_GRAD_SHIFT) return backward_shift(t, lam_T, lam0, grad_v, s);
   // Partial-sum scratch of the adjoint kernel, sized for every buffer
   // pairing the sweep uses (f_t is always a tape buffer).
@@ -717,6 +710,34 @@ int fdb_tape_backward(fdb_tape_t* t, const void* lam_T, void* lam0, double* grad
   // forward.
   t->forward_done = false;
   return FDB_OK;
+}
+
+// A call that fails after its first launch still returns with its work done:
+// the caller's workspace and fields may be freed at once.
+int finish(int rc, hipStream_t s) {
+  if (rc != FDB_OK) (void)hipStreamSynchronize(s);
+  return rc;
+}
+
+}  // namespace
+
+extern "C" {
+
+int fdb_tape_forward(fdb_tape_t* t, const void* f0, void* fT, void* stream) {
+  if (!t || !f0 || !fT) return tfail(FDB_ERR_INVALID, "tape_forward: null argument");
+  if (f0 == fT) return tfail(FDB_ERR_INVALID, "tape_forward: f0 and fT must differ");
+  if (t->external && !t->ws_set) return tfail(FDB_ERR_INVALID, "tape_forward: no workspace set");
+  return finish(forward_run(t, f0, fT, (hipStream_t)stream), (hipStream_t)stream);
+}
+
+int fdb_tape_backward(fdb_tape_t* t, const void* lam_T, void* lam0, double* grad_v,
+                      void* stream) {
+  if (!t || !lam_T || !lam0 || !grad_v)
+    return tfail(FDB_ERR_INVALID, "tape_backward: null argument");
+  if (lam_T == lam0) return tfail(FDB_ERR_INVALID, "tape_backward: lam_T and lam0 must differ");
+  if (!t->forward_done) return tfail(FDB_ERR_INVALID, "tape_backward: run tape_forward first");
+  if (t->external && !t->ws_set) return tfail(FDB_ERR_INVALID, "tape_backward: no workspace set");
+  return finish(backward_run(t, lam_T, lam0, grad_v, (hipStream_t)stream), (hipStream_t)stream);
 }
 
 int fdb_tape_set_time_block(fdb_tape_t* t, int k) {
