@@ -106,6 +106,9 @@ bool plane_pass_supported(int dtype, const Grid3& g, int k);
 // hipErrorNotSupported unless plane_pass_supported; src is only read.
 hipError_t launch_plane_pass(int dtype, const Grid3& g, const void* src, void* dst, int k,
                              hipStream_t s);
+// Whether a one-step launch over g is plane_kernel's: where it is supported
+// and no FDB_ROWS_CFG variable asks for a shape of the rows kernel.
+bool one_step_by_plane(int dtype, const Grid3& g);
 // Modelled time (us) of one k-step launch over the 2-D grid g.
 float plane_pass_us(int dtype, const Grid3& g, int k);
 

@@ -2351,6 +2351,10 @@ int plan_pass(int dtype, const Grid3& g, int left, int cap) {
   return first[left];
 }
 
+bool one_step_by_plane(int dtype, const Grid3& g) {
+  return plane_pass_supported(dtype, g, 1) && !tuning().rows_env[0][dtype_size(dtype)][0];
+}
+
 const char* tuning_error() {
   const Tuning& t = tuning();
   return t.error.empty() ? nullptr : t.error.c_str();
@@ -2403,7 +2407,7 @@ hipError_t launch_advect_pass(int dtype, const Grid3& g, void* const bufs[2], in
       }
       if (err != hipErrorNotSupported) return err;
     }
-    if (done == 0 && plane_pass_supported(dtype, g, 1)) {
+    if (done == 0 && one_step_by_plane(dtype, g)) {
       err = launch_plane_pass(dtype, g, src, dst, 1, s);
       if (err != hipSuccess) return err;
       done = 1;

@@ -14,6 +14,7 @@
 //
 //   san_host            the checks above
 //   san_host tuning     the same process with malformed tuning variables set
+//   san_host rows       ... with a shape for the FP64 rows kernel set
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
@@ -253,6 +254,20 @@ void constructors() {
   check(rc == FDB_ERR_NODEV || (rc == FDB_OK && fdb_upwind_destroy(h) == FDB_OK), "create nodev");
 }
 
+// Which one-step launches over a 2-D field the plane kernel makes; rows_64:
+// FDB_ROWS_CFG_8 is set.
+void one_step_routes(bool rows_64) {
+  const uint64_t n[3] = {40, 50, 60};
+  const double v[3] = {0.3, -0.2, 0.1}, len[3] = {1, 1, 1};
+  fdb::Grid3 g2, g3;
+  check(fdb::make_grid(2, n, v, len, 1e-3, &g2) && fdb::make_grid(3, n, v, len, 1e-3, &g3), "grid");
+  check(fdb::one_step_by_plane(FDB_F64, g2) == !rows_64, "2-D FP64 step");
+  check(fdb::one_step_by_plane(FDB_F32, g2), "2-D FP32 step");
+  check(!fdb::one_step_by_plane(FDB_BF16, g2) && !fdb::one_step_by_plane(FDB_BF16_SR, g2),
+        "2-D bf16 step");
+  check(!fdb::one_step_by_plane(FDB_F64, g3), "3-D step");
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -269,7 +284,11 @@ int main(int argc, char** argv) {
     fdb_tape_t* t = nullptr;
     check(fdb_tape_create(3, ok, v, len, 0.01, 4, FDB_F64, FDB_F64, 1 << 30, &t) ==
               FDB_ERR_INVALID, "tuning refused (tape)");
+  } else if (argc > 1 && std::strcmp(argv[1], "rows") == 0) {
+    setenv("FDB_ROWS_CFG_8", "4,2,0,1", 1);
+    one_step_routes(true);
   } else {
+    one_step_routes(false);
     plans();
     folds_and_vtk();
     fold_maps();
@@ -281,6 +300,6 @@ int main(int argc, char** argv) {
     std::fprintf(stderr, "%d check(s) failed\n", g_fail);
     return 1;
   }
-  std::printf("san_host ok%s\n", argc > 1 ? " (tuning)" : "");
+  std::printf("san_host ok%s%s\n", argc > 1 ? " " : "", argc > 1 ? argv[1] : "");
   return 0;
 }

@@ -33,3 +33,10 @@ def test_host_code_is_clean_under_asan_and_ubsan(san_host, mode, tmp_path):
     assert p.returncode == 0, p.stdout[-2000:] + p.stderr[-4000:]
     assert "san_host ok" in p.stdout
     assert "ERROR: AddressSanitizer" not in p.stderr and "runtime error" not in p.stderr
+
+
+def test_rows_variable_reaches_two_dimensional_steps(san_host):
+    """With FDB_ROWS_CFG_8 set, one-step launches over 2-D FP64 fields are the
+    rows kernel's again; other types' are not touched."""
+    p = subprocess.run([san_host, "rows"], capture_output=True, text=True, timeout=600)
+    assert p.returncode == 0 and "san_host ok rows" in p.stdout, p.stderr[-2000:]
