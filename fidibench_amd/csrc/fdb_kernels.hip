@@ -1595,6 +1595,19 @@ RowsCfg rows_cfg(int bytes, bool adj, int fbytes, int64_t ntot) {
   return c;
 }
 
+// Cells per lane of the rows kernel, from at most vec: narrowed while that
+// leaves fewer idle lanes in a row's last tile (a 768-cell bf16 row takes two
+// 512-cell tiles at 8 cells per lane, a quarter of the lanes idle, but three
+// exact tiles at 4).
+int fill_lanes(int64_t n2, int vec) {
+  auto idle = [&](int v) {
+    const int64_t w = 64 * (int64_t)v;
+    return ((n2 + w - 1) / w) * w - n2;
+  };
+  while (vec > 1 && idle(vec / 2) < idle(vec)) vec >>= 1;
+  return vec;
+}
+
 // Launches the rows kernel for one step (forward: dirs = u, adjoint:
 // dirs = -u).  With dry = true only reports the block count.
 template <typename TS, typename TF, bool ADJ, bool SR = false>
@@ -1623,14 +1636,7 @@ hipError_t rows_dispatch(const Grid3& g, const TS* in, TS* out, const int dirs[3
   while (vec > 1 && ((a.n2 % vec) != 0 || (align_bits % (vec * sizeof(TS))) != 0 ||
                      ((uintptr_t)ft % (vec * sizeof(TF))) != 0))
     vec >>= 1;
-  // ... narrowed while that leaves fewer idle lanes in a row's last tile
-  // (a 768-cell bf16 row takes two 512-cell tiles at 8 cells per lane, a
-  // quarter of the lanes idle, but three exact tiles at 4).
-  auto idle = [&](int v) {
-    const int64_t w = 64 * (int64_t)v;
-    return ((a.n2 + w - 1) / w) * w - a.n2;
-  };
-  while (vec > 1 && idle(vec / 2) < idle(vec)) vec >>= 1;
+  vec = fill_lanes(a.n2, vec);
   a.tiles2 = (a.n2 + 64 * vec - 1) / (64 * vec);
   auto tiles1 = [&] { return (a.n1 + (int64_t)cfg.WY * cfg.R - 1) / ((int64_t)cfg.WY * cfg.R); };
   // The products' partial slots stay within 65536 (up to 4 chunks per
@@ -2138,6 +2144,21 @@ bool make_grid(int ndims, const uint64_t* n, const double* v, const double* len,
   return true;
 }
 
+float rows_step_us(int dtype, const Grid3& g) {
+  const int bytes = (int)dtype_size(dtype);
+  int vec = 16 / bytes;
+  while (vec > 1 && g.n[2] % vec != 0) vec >>= 1;
+  vec = fill_lanes(g.n[2], vec);
+  const double tiles = (double)(g.ntot / g.n[2] * ((g.n[2] + 64 * vec - 1) / (64 * vec)));
+  // ns per row tile: fixed, and per cell of a lane.
+  static constexpr double k64[2] = {0.115, 0.033}, k32[2] = {0.013, 0.074},
+                          k16[2] = {0.045, 0.046}, ksr[2] = {0.033, 0.070};
+  const double* k = bytes == 8 ? k64 : (bytes == 4 ? k32 : (dtype == FDB_BF16_SR ? ksr : k16));
+  const double moved = 2.0 * (double)g.ntot * bytes;
+  const double mem = moved / (moved <= (double)kResidentBytes ? 6.6e6 : 5.2e6);
+  return (float)(3.6 + std::max(mem, 1e-3 * tiles * (k[0] + k[1] * vec)));
+}
+
 bool fused_pass_supported(int dtype, const Grid3& g, int k) {
   if (k < 2 || k > kMaxTimeBlock) return false;
   if (is_plane(g)) return plane_pass_supported(dtype, g, k);
@@ -2245,10 +2266,7 @@ PassCosts pass_costs(int dtype, const Grid3& g) {
     return c;
   }
   if (cells < 1.0 && dtype != FDB_BF16_SR) {
-    // One step: a launch, then its fields at the rate of the Infinity Cache
-    // or of HBM (64^3 to 384^3, all types, within 25 %).
-    const double bytes = 2.0 * (double)g.ntot * (double)dtype_size(dtype);
-    c.us[1] = (float)(3.6 + bytes / (bytes <= (double)kResidentBytes ? 6.6e6 : 5.2e6));
+    c.us[1] = rows_step_us(dtype, g);
     const PassPicks p = pass_picks((int)dtype_size(dtype), g);
     for (int k = 2; k <= kMaxTimeBlock; ++k) {
       if (!fused_pass_supported(dtype, g, k)) continue;

@@ -363,11 +363,12 @@ hipError_t launch_plane_pass(int dtype, const Grid3& g, const void* src, void* d
 float plane_pass_us(int dtype, const Grid3& g, int k) {
   const double bytes = 2.0 * (double)g.ntot * (double)dtype_size(dtype);
   const bool resident = bytes <= (double)(256ll << 20);
-  if (k == 1) {
-    if (dtype != FDB_F64 && dtype != FDB_F32) return (float)(3.5 + bytes / 5.0e6);
-    return (float)(3.0 + bytes / (resident ? 8.3e6 : 5.7e6));
-  }
+  if (k == 1 && dtype != FDB_F64 && dtype != FDB_F32) return rows_step_us(dtype, g);
   const PlaneArgs a = plane_args(g, k);
+  if (k == 1) {  // ns per wave: 2077634 x 3, 1219781 x 1, 199464 x 3 (297, 175, 33 us FP64)
+    const double waves = 1e-3 * (double)a.ntiles * (dtype == FDB_F64 ? 0.43 : 0.35);
+    return (float)(3.0 + std::max(waves, bytes / (resident ? 8.3e6 : 5.7e6)));
+  }
   const double level = dtype == FDB_F64 ? 0.0285 : (dtype == FDB_F32 ? 0.021 : 0.026);
   const double waves = (double)a.ntiles / (double)kWaveSlots;
   // (More than four waves per SIMD hide each other's latency: FP32 8000 x

@@ -1,0 +1,31 @@
+"""The planner over grids whose rows are short: a one-step launch costs by the
+rows it issues there, not by its bytes, and several steps a launch are cheaper
+(launch times measured on MI355X)."""
+from __future__ import annotations
+
+import pytest
+
+
+def _passes(dtype, shape, nsteps=22):
+    from fidibench_amd import _lib as L
+    v = (0.4, -0.3, 0.35)[:len(shape)]
+    return L.plan_passes(shape, v, (1.0,) * len(shape), 1e-6, getattr(L, dtype), nsteps, 0)
+
+
+@pytest.mark.parametrize("dtype,shape", [
+    ("F64", (1256, 3519, 2)),   # us a step, one a launch / fused: 537 / 127
+    ("F32", (1256, 3519, 2)),   # 313 / 68
+    ("BF16", (1256, 3519, 2)),  # 339 / 86
+    ("F64", (200, 300, 1)),     # 10.9 / 2.6
+    ("F32", (74, 6433, 9)),     # 56 / 13
+    ("BF16", (400, 400, 16)),   # 16.7 / 4.1
+    ("BF16", (300507, 14)),     # 62 / 9
+    ("F32", (2077634, 3)),      # 243 / 44
+])
+def test_short_rows_take_several_steps_a_launch(dtype, shape):
+    assert 1 not in _passes(dtype, shape)
+
+
+@pytest.mark.parametrize("dtype", ["F64", "F32", "BF16"])
+def test_one_step_in_one_launch(dtype):
+    assert _passes(dtype, (1256, 3519, 2), 1) == [1]
