@@ -109,6 +109,9 @@ hipError_t launch_plane_pass(int dtype, const Grid3& g, const void* src, void* d
 // Whether a one-step launch over g is plane_kernel's: where it is supported
 // and no FDB_ROWS_CFG variable asks for a shape of the rows kernel.
 bool one_step_by_plane(int dtype, const Grid3& g);
+// Planes per tile that the model picks for a k-step fused pass over a 3-D grid
+// of less than 512^3 cells, and the rows of its blocks (for the CPU tests).
+int64_t picked_chunk(int dtype, const Grid3& g, int k, int* rows);
 // Modelled time (us) of one step by the rows kernel, below 512^3 cells: a
 // launch, then its fields at the rate of the Infinity Cache or of HBM, or its
 // row tiles (64 lanes x up to 16 bytes of a row) at the rate they issue, which

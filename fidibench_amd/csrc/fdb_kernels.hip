@@ -1796,12 +1796,20 @@ struct PassPick {
   double us = 0.0;  // 0: no pick
 };
 
-// Calls f(chunk) for the candidate planes per tile of n0 planes.
+// Calls f(chunk) for the candidate planes per tile of n0 planes, the device
+// holding cap blocks of tiles each: up to 24 planes; above that 1 to 16 chunks,
+// then counts a sixteenth apart, and the counts that fill one to four rounds of
+// blocks (3088 x 19 x 404 FP64, 7 steps, 8 tiles of one block per CU: 32
+// chunks, 281 us, where 24 take 375).
 template <class F>
-void for_chunks(int64_t n0, F f) {
+void for_chunks(int64_t n0, int64_t tiles, int64_t cap, F f) {
   for (int64_t c = 1; c <= std::min<int64_t>(24, n0); ++c) f(c);
-  for (int64_t nch = 1; nch <= 24; ++nch)
-    if ((n0 + nch - 1) / nch > 24) f((n0 + nch - 1) / nch);
+  for (int64_t nch = 1; (n0 + nch - 1) / nch > 24; nch += std::max<int64_t>(1, nch / 16))
+    f((n0 + nch - 1) / nch);
+  for (int64_t round = 1; round <= 4; ++round) {
+    const int64_t nch = round * cap / tiles;
+    if (nch >= 1 && nch <= n0) f((n0 + nch - 1) / nch);
+  }
 }
 
 // The model's time of a pass's arithmetic, us, without its launch: rounds
@@ -1832,7 +1840,7 @@ PassPick pick_pass(int bytes, const Grid3& g, int K) {
     if (s.K != K || occ == 0 || s.WY * s.R <= K) continue;
     const int64_t tiles = ((g.n[2] + (64 - K) - 1) / (64 - K)) *
                           ((g.n[1] + (s.WY * s.R - K) - 1) / (s.WY * s.R - K));
-    for_chunks(n0, [&](int64_t chunk) {
+    for_chunks(n0, tiles, 256 * (int64_t)occ, [&](int64_t chunk) {
       double t = pass_compute(m, s.R, s.WY, K, tiles, n0, chunk, occ);
       t = m.launch + std::cbrt(t * t * t + mem * mem * mem);
       if (best.us == 0.0 || t < best.us) best = PassPick{TbCfg{s.R, s.WY, 0}, chunk, t};
@@ -1849,7 +1857,7 @@ PassPick pick_pass(int bytes, const Grid3& g, int K) {
 int64_t adj_chunk(int bytes, int R, int WY, int K, int64_t tiles, int64_t n0, int64_t occ) {
   int64_t best = n0;
   double least = -1.0;
-  for_chunks(n0, [&](int64_t chunk) {
+  for_chunks(n0, tiles, 256 * occ, [&](int64_t chunk) {
     const double t = pass_compute(pass_model(bytes), R, WY, K, tiles, n0, chunk, occ);
     if (least < 0.0 || t < least) {
       least = t;
@@ -2367,6 +2375,12 @@ int plan_pass(int dtype, const Grid3& g, int left, int cap) {
     }
   }
   return first[left];
+}
+
+int64_t picked_chunk(int dtype, const Grid3& g, int k, int* rows) {
+  const PassPick p = pass_picks((int)dtype_size(dtype), g).k[k];
+  if (rows) *rows = p.cfg.R * p.cfg.WY;
+  return p.chunk;
 }
 
 bool one_step_by_plane(int dtype, const Grid3& g) {

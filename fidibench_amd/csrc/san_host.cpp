@@ -268,6 +268,30 @@ void one_step_routes(bool rows_64) {
   check(!fdb::one_step_by_plane(FDB_F64, g3), "3-D step");
 }
 
+// The tiles of fused passes over long grids fill the device: 8 tiles an axis-0
+// chunk, one block per CU, where 1 to 24 chunks leave a quarter of it idle.
+void long_grid_chunks() {
+  const uint64_t n[3] = {3088, 19, 404};
+  const double v[3] = {0.3, -0.2, 0.1}, len[3] = {1, 1, 1};
+  fdb::Grid3 g;
+  check(fdb::make_grid(3, n, v, len, 1e-3, &g), "grid");
+  int rows = 0;
+  const int64_t chunk = fdb::picked_chunk(FDB_F64, g, 7, &rows);
+  check(chunk > 0 && rows > 7, "a pick");
+  const int64_t tiles = (404 + 56) / 57 * ((19 + rows - 8) / (rows - 7));
+  const int64_t blocks = tiles * ((3088 + chunk - 1) / chunk);
+  check(blocks % 256 == 0 || blocks % 256 > 224, "blocks fill the last round");
+  // Every grid gets a chunk within its planes.
+  for (uint64_t n0 : {1, 2, 23, 24, 25, 600, 601, 5000, 1000000})
+    for (int dt : {FDB_F64, FDB_F32, FDB_BF16})
+      for (int k : {2, 3, 4, 6, 7, 8}) {
+        const uint64_t m[3] = {n0, 3, 5};
+        check(fdb::make_grid(3, m, v, len, 1e-3, &g), "grid");
+        const int64_t c = fdb::picked_chunk(dt, g, k, nullptr);
+        check(c >= 1 && c <= (int64_t)n0, "chunk within the planes");
+      }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -289,6 +313,7 @@ int main(int argc, char** argv) {
     one_step_routes(true);
   } else {
     one_step_routes(false);
+    long_grid_chunks();
     plans();
     folds_and_vtk();
     fold_maps();
