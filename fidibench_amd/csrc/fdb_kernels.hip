@@ -1777,18 +1777,20 @@ const PassModel& pass_model(int bytes) {
   return bytes == 8 ? m64 : (bytes == 4 ? m32 : m16);
 }
 
-// Shapes to pick from, by depth, with the blocks a CU holds of each (FP64;
-// FP32 and bf16).  Measured at 96^3 FP64, us per launch: K = 4 with 2, 4
-// and 9 rows 9.2, 10.1, 12.2; K = 6 with 4, 8 and 9 rows 15.3, 22.9, 26.1;
-// 256^3: K = 6 with 4 and 8 rows 75.5, 83.4.  (FP32 K = 6 with 4 rows is
-// left out: it is no faster per step than K = 4 with 6.)
+// Shapes to pick from, by depth, with the blocks a CU holds of each (FP64,
+// FP32, bf16; 0: not for this type).  Measured at 96^3 FP64, us per launch:
+// K = 4 with 2, 4 and 9 rows 9.2, 10.1, 12.2; K = 6 with 4, 8 and 9 rows 15.3,
+// 22.9, 26.1; 256^3: K = 6 with 4 and 8 rows 75.5, 83.4.  (FP32 K = 6 with 4
+// rows is left out: it is no faster per step than K = 4 with 6.)  bf16 K = 6
+// with 9 rows takes 130 VGPRs, one block per CU: 256^3 92 us, with 8 rows 72.
 struct PassShape {
-  int K, R, WY, occ64, occ32;
+  int K, R, WY, occ64, occ32, occ16;
 };
 constexpr PassShape kPassShapes[] = {
-    {2, 2, 8, 4, 4}, {2, 9, 4, 4, 8}, {3, 2, 8, 4, 4}, {3, 9, 4, 3, 6}, {4, 2, 8, 4, 4},
-    {4, 4, 8, 3, 0}, {4, 6, 8, 0, 4}, {4, 9, 4, 3, 5}, {6, 4, 8, 2, 0}, {6, 8, 8, 1, 2},
-    {6, 9, 8, 1, 2}, {7, 8, 8, 1, 0}, {7, 9, 8, 0, 2}, {8, 9, 8, 1, 2}};
+    {2, 2, 8, 4, 4, 4}, {2, 9, 4, 4, 8, 8}, {3, 2, 8, 4, 4, 4}, {3, 9, 4, 3, 6, 6},
+    {4, 2, 8, 4, 4, 4}, {4, 4, 8, 3, 0, 0}, {4, 6, 8, 0, 4, 4}, {4, 9, 4, 3, 5, 5},
+    {6, 4, 8, 2, 0, 0}, {6, 8, 8, 1, 2, 2}, {6, 9, 8, 1, 2, 1}, {7, 8, 8, 1, 0, 0},
+    {7, 9, 8, 0, 2, 2}, {8, 9, 8, 1, 2, 2}};
 
 struct PassPick {
   TbCfg cfg{0, 0, 0};
@@ -1836,7 +1838,7 @@ PassPick pick_pass(int bytes, const Grid3& g, int K) {
   const int64_t n0 = g.n[0];
   const double mem = 2.0 * (double)g.ntot * bytes / m.bw;
   for (const PassShape& s : kPassShapes) {
-    const int occ = bytes == 8 ? s.occ64 : s.occ32;
+    const int occ = bytes == 8 ? s.occ64 : (bytes == 4 ? s.occ32 : s.occ16);
     if (s.K != K || occ == 0 || s.WY * s.R <= K) continue;
     const int64_t tiles = ((g.n[2] + (64 - K) - 1) / (64 - K)) *
                           ((g.n[1] + (s.WY * s.R - K) - 1) / (s.WY * s.R - K));

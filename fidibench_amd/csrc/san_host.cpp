@@ -268,6 +268,21 @@ void one_step_routes(bool rows_64) {
   check(!fdb::one_step_by_plane(FDB_F64, g3), "3-D step");
 }
 
+// Rows of a k-step launch's blocks.
+int picked_rows(int dtype, uint64_t n0, uint64_t n1, uint64_t n2, int k) {
+  const uint64_t n[3] = {n0, n1, n2};
+  const double v[3] = {0.3, -0.2, 0.1}, len[3] = {1, 1, 1};
+  fdb::Grid3 g;
+  check(fdb::make_grid(3, n, v, len, 1e-3, &g), "grid");
+  int rows = 0;
+  check(fdb::picked_chunk(dtype, g, k, &rows) > 0, "a pick");
+  return rows;
+}
+
+void picked_shapes() {
+  check(picked_rows(FDB_BF16, 256, 256, 256, 6) == 64, "bf16 6 steps: two blocks per CU");
+}
+
 // The tiles of fused passes over long grids fill the device: 8 tiles an axis-0
 // chunk, one block per CU, where 1 to 24 chunks leave a quarter of it idle.
 void long_grid_chunks() {
@@ -314,6 +329,7 @@ int main(int argc, char** argv) {
   } else {
     one_step_routes(false);
     long_grid_chunks();
+    picked_shapes();
     plans();
     folds_and_vtk();
     fold_maps();
