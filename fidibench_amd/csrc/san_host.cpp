@@ -281,6 +281,9 @@ int picked_rows(int dtype, uint64_t n0, uint64_t n1, uint64_t n2, int k) {
 
 void picked_shapes() {
   check(picked_rows(FDB_BF16, 256, 256, 256, 6) == 64, "bf16 6 steps: two blocks per CU");
+  check(picked_rows(FDB_F64, 158, 102, 177, 2) == 36, "FP64 2 steps: tall waves");
+  check(picked_rows(FDB_F32, 13, 1794, 12, 2) == 36, "FP32 2 steps: tall waves");
+  check(picked_rows(FDB_F64, 16, 16, 16, 4) == 16, "FP64 4 steps: short waves");
 }
 
 // The tiles of fused passes over long grids fill the device: 8 tiles an axis-0
