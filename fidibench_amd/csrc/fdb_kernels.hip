@@ -1783,6 +1783,7 @@ const PassModel& pass_model(int bytes) {
 // 22.9, 26.1; 256^3: K = 6 with 4 and 8 rows 75.5, 83.4.  (FP32 K = 6 with 4
 // rows is left out: it is no faster per step than K = 4 with 6.)  bf16 K = 6
 // with 9 rows takes 130 VGPRs, one block per CU: 256^3 92 us, with 8 rows 72.
+// FP64 K = 8 with 7 and 9 rows: 3088x19x404 276 and 370 us, 300x310x290 175 and 192.
 struct PassShape {
   int K, R, WY, occ64, occ32, occ16;
 };
@@ -1790,7 +1791,7 @@ constexpr PassShape kPassShapes[] = {
     {2, 2, 8, 4, 4, 4}, {2, 9, 4, 4, 8, 8}, {3, 2, 8, 4, 4, 4}, {3, 9, 4, 3, 6, 6},
     {4, 2, 8, 4, 4, 4}, {4, 4, 8, 3, 0, 0}, {4, 6, 8, 0, 4, 4}, {4, 9, 4, 3, 5, 5},
     {6, 4, 8, 2, 0, 0}, {6, 8, 8, 1, 2, 2}, {6, 9, 8, 1, 2, 1}, {7, 8, 8, 1, 0, 0},
-    {7, 9, 8, 0, 2, 2}, {8, 9, 8, 1, 2, 2}};
+    {7, 9, 8, 0, 2, 2}, {8, 7, 8, 1, 0, 0}, {8, 9, 8, 1, 2, 2}};
 
 struct PassPick {
   TbCfg cfg{0, 0, 0};

@@ -284,6 +284,7 @@ void picked_shapes() {
   check(picked_rows(FDB_F64, 158, 102, 177, 2) == 36, "FP64 2 steps: tall waves");
   check(picked_rows(FDB_F32, 13, 1794, 12, 2) == 36, "FP32 2 steps: tall waves");
   check(picked_rows(FDB_F64, 16, 16, 16, 4) == 16, "FP64 4 steps: short waves");
+  check(picked_rows(FDB_F64, 3088, 19, 404, 8) == 56, "FP64 8 steps: two planes a trip");
 }
 
 // The tiles of fused passes over long grids fill the device: 8 tiles an axis-0
