@@ -1768,6 +1768,7 @@ struct PassModel {
   double rate[4];     // ns per instruction and wave, 1..4 waves per SIMD
   double sync, row;   // us per level; instructions per row and plane
   double bw;          // MB per us
+  double plane = 0.0; // us per plane
 };
 constexpr int64_t kModelCells = 1ll << 27;
 const PassModel& pass_model(int bytes) {
@@ -1830,7 +1831,8 @@ double pass_compute(const PassModel& m, int R, int WY, int K, int64_t tiles, int
     const double x = std::min(4.0, std::max(1.0, w)) - 1.0;
     const int i = std::min(2, (int)x);
     const double rate = m.rate[i] + (x - i) * (m.rate[i + 1] - m.rate[i]);
-    return w * R * (11.0 * K + m.row) * (R == 2 ? kTwoRows : 1.0) * rate * 1e-3 + K * m.sync;
+    return w * R * (11.0 * K + m.row) * (R == 2 ? kTwoRows : 1.0) * rate * 1e-3 + K * m.sync +
+           m.plane;
   };
   const int64_t blocks = tiles * ((n0 + chunk - 1) / chunk);
   const int64_t cap = occ * 256, full = blocks / cap, rest = blocks - full * cap;
@@ -1874,6 +1876,21 @@ int64_t adj_chunk(int bytes, int R, int WY, int K, int64_t tiles, int64_t n0, in
     }
   });
   return best;
+}
+
+// The same for a stochastic-rounding pass (K = 2, 4 or 8; its shape pairs rows
+// and is fixed, its chunks fill the device: tb_dispatch).  Constants fitted to
+// 213 launches over 127 grids, rms error 5 %.
+double sr_pass_us(const Grid3& g, int K) {
+  static constexpr PassModel m = {3.81, {1.68, 1.68, 1.63, 1.72}, 0.096, 10.4, 4.6e6, 0.271};
+  const TbCfg c = tb_sr_cfg(K);
+  const int64_t occ = K == 2 ? 7 : (K == 4 ? 5 : 2), n0 = g.n[0];
+  const int64_t tiles = ((g.n[2] + (64 - K) - 1) / (64 - K)) *
+                        ((g.n[1] + (c.WY * c.R - K) - 1) / (c.WY * c.R - K));
+  const int64_t nch = march_chunks(tiles, n0, K, occ * 256, 1, 64, true);
+  const double t = pass_compute(m, c.R, c.WY, K, tiles, n0, (n0 + nch - 1) / nch, occ);
+  const double mem = 4.0 * (double)g.ntot / m.bw;
+  return m.launch + std::cbrt(t * t * t + mem * mem * mem);
 }
 
 // The picks of every depth for the last few (type, grid) pairs.
@@ -2169,7 +2186,7 @@ float rows_step_us(int dtype, const Grid3& g) {
   const double tiles = (double)(g.ntot / g.n[2] * ((g.n[2] + 64 * vec - 1) / (64 * vec)));
   // ns per row tile: fixed, and per cell of a lane.
   static constexpr double k64[2] = {0.115, 0.033}, k32[2] = {0.013, 0.074},
-                          k16[2] = {0.045, 0.046}, ksr[2] = {0.033, 0.070};
+                          k16[2] = {0.045, 0.046}, ksr[2] = {0.033, 0.068};
   const double* k = bytes == 8 ? k64 : (bytes == 4 ? k32 : (dtype == FDB_BF16_SR ? ksr : k16));
   const double moved = 2.0 * (double)g.ntot * bytes;
   const double mem = moved / (moved <= (double)kResidentBytes ? 6.6e6 : 5.2e6);
@@ -2202,15 +2219,6 @@ constexpr float kPassUs[4][kMaxTimeBlock + 1] = {
     {0, 373, 573, 576, 537, 0, 549, 577, 705},
     {0, 190, 331, 333, 333, 0, 344, 381, 378},
     {0, 99, 163, 172, 217, 0, 402, 320, 416},
-    {0, 115, 167, 0, 325, 0, 0, 0, 729}};
-// Stochastic rounding on cubic grids of kSrSide[i]^3 cells (its passes
-// pair rows, so their shapes do not follow the grid).
-constexpr int kSrSizes = 4;
-constexpr double kSrSide[kSrSizes] = {16, 128, 256, 512};
-constexpr float kSrUsAt[kSrSizes][kMaxTimeBlock + 1] = {
-    {0, 3.9f, 6.7f, 0, 10.5f, 0, 0, 0, 37.7f},
-    {0, 5.9f, 13.5f, 0, 24.8f, 0, 0, 0, 76.4f},
-    {0, 19.2f, 33.0f, 0, 64.0f, 0, 0, 0, 140.0f},
     {0, 115, 167, 0, 325, 0, 0, 0, 729}};
 constexpr int kPlanTail = 48;  // steps split exactly; longer runs first take the best depth
 int pass_row(int dtype) {
@@ -2248,8 +2256,7 @@ int64_t fused_pass_visits(int dtype, const Grid3& g, int k) {
 // equal time per plane there, so the length captures rounds of resident
 // blocks, warm-up planes and tiles cut by the grid's extents; at 1024^3 FP64
 // this picks 8-step passes, 679 us per step, over 7-step ones, 710).  On
-// smaller grids the pass's own model (pick_pass) and, for stochastic
-// rounding, measured times (below 16^3 cells those of 16^3).
+// smaller grids the pass's own model (pick_pass, sr_pass_us).
 struct PassCosts {
   float us[kMaxTimeBlock + 1];
 };
@@ -2282,29 +2289,15 @@ PassCosts pass_costs(int dtype, const Grid3& g) {
       if (k == 1 || plane_pass_supported(dtype, g, k)) c.us[k] = plane_pass_us(dtype, g, k);
     return c;
   }
-  if (cells < 1.0 && dtype != FDB_BF16_SR) {
+  if (cells < 1.0) {
     c.us[1] = rows_step_us(dtype, g);
-    const PassPicks p = pass_picks((int)dtype_size(dtype), g);
+    const bool sr = dtype == FDB_BF16_SR;
+    const PassPicks p = sr ? PassPicks{} : pass_picks((int)dtype_size(dtype), g);
     for (int k = 2; k <= kMaxTimeBlock; ++k) {
       if (!fused_pass_supported(dtype, g, k)) continue;
-      c.us[k] = (float)p.k[k].us;
-      if (p.k[k].us <= 0.0 && kPassUs[row][k] > 0.0f)  // a shape set by a tuning variable
+      c.us[k] = (float)(sr ? sr_pass_us(g, k) : p.k[k].us);
+      if (!sr && p.k[k].us <= 0.0 && kPassUs[row][k] > 0.0f)  // a shape set by a tuning variable
         c.us[k] = (float)(4.0 + kPassUs[row][k] * cells);
-    }
-    return c;
-  }
-  if (cells < 1.0) {
-    // Stochastic rounding: between the measured sizes i and i + 1, linearly
-    // in log(time) against log(cells).
-    const double lc = std::log((double)g.ntot);
-    int i = 0;
-    while (i + 2 < kSrSizes && lc > 3.0 * std::log(kSrSide[i + 1])) ++i;
-    const double l0 = 3.0 * std::log(kSrSide[i]), l1 = 3.0 * std::log(kSrSide[i + 1]);
-    const double a = std::min(1.0, std::max(0.0, (lc - l0) / (l1 - l0)));
-    for (int k = 1; k <= kMaxTimeBlock; ++k) {
-      const float t0 = kSrUsAt[i][k], t1 = kSrUsAt[i + 1][k];
-      if (t0 <= 0.0f || t1 <= 0.0f || (k > 1 && !fused_pass_supported(dtype, g, k))) continue;
-      c.us[k] = (float)std::exp((1.0 - a) * std::log((double)t0) + a * std::log((double)t1));
     }
     return c;
   }

@@ -29,3 +29,16 @@ def test_short_rows_take_several_steps_a_launch(dtype, shape):
 @pytest.mark.parametrize("dtype", ["F64", "F32", "BF16"])
 def test_one_step_in_one_launch(dtype):
     assert _passes(dtype, (1256, 3519, 2), 1) == [1]
+
+
+@pytest.mark.parametrize("shape,deep", [
+    ((104, 48, 225), True),     # us a step, one a launch / 4-step passes: 6.3 / 4.4
+    ((1, 554, 2013), True),     # 7.2 / 4.8
+    ((290, 38, 222), True),     # 8.4 / 5.7
+    ((192, 3014, 2), True),     # 51 / 24
+    ((1462, 4, 2), False),      # 5.2 / 9.8
+    ((1643, 2, 2), False),      # 6.1 / 10.4
+])
+def test_stochastic_rounding_follows_the_grid_not_its_cells(shape, deep):
+    ks = _passes("BF16_SR", shape)
+    assert (1 not in ks) if deep else set(ks) == {1}, ks
