@@ -112,6 +112,8 @@ bool one_step_by_plane(int dtype, const Grid3& g);
 // Planes per tile that the model picks for a k-step fused pass over a 3-D grid
 // of less than 512^3 cells, and the rows of its blocks (for the CPU tests).
 int64_t picked_chunk(int dtype, const Grid3& g, int k, int* rows);
+// Waves of a block of the rows kernel's forward step (for the CPU tests).
+int one_step_waves(int dtype, const Grid3& g);
 // Modelled time (us) of one step by the rows kernel, below 512^3 cells: a
 // launch, then its fields at the rate of the Infinity Cache or of HBM, or its
 // row tiles (64 lanes x up to 16 bytes of a row) at the rate they issue, which

@@ -1581,16 +1581,20 @@ const Tuning& tuning() {
   return t;
 }
 
-// The shape for a step over ntot cells (kResidentBytes: the small fields').
-RowsCfg rows_cfg(int bytes, bool adj, int fbytes, int64_t ntot) {
+// The shape for a step over ntot cells in planes of n1 rows (kResidentBytes:
+// the small fields').  Up to four rows leave two of that shape's four waves
+// without any: two waves then, us a step with four / two (8 x 2, 4 x 2 before
+// them): 1-D 3000001 FP64 82 / 45 (159), FP32 75 / 40 (55); 100 x 2 x 4000 FP64
+// 9.5 / 7.8; 1 x 4 x 700001 FP32 21.5 / 13.0; (1 x 8 x 300000 FP64 10.4 / 10.8).
+RowsCfg rows_cfg(int bytes, bool adj, int fbytes, int64_t ntot, int64_t n1) {
   const Tuning& t = tuning();
   const int a = adj ? 1 : 0, fb = adj ? fbytes : 0;
   RowsCfg c = t.rows[a][bytes][fb];
   const int64_t cell = 2 * bytes + fb;
   if (!t.rows_env[a][bytes][fb] && ntot <= kResidentBytes / cell) {
     c.R = 2;
-    c.WY = 4;
-    c.nt = ntot <= kCachedStoreBytes / cell ? 1 : 0;
+    c.WY = n1 <= 4 ? 2 : 4;
+    c.nt = n1 <= 4 || ntot <= kCachedStoreBytes / cell ? 1 : 0;
   }
   return c;
 }
@@ -1615,7 +1619,7 @@ hipError_t rows_dispatch(const Grid3& g, const TS* in, TS* out, const int dirs[3
                          const TF* ft, double* partials, int64_t* nblocks_out, hipStream_t s,
                          bool dry, uint32_t sr_key = 0) {
   using M = typename St<TS>::M;
-  RowsCfg cfg = rows_cfg((int)sizeof(TS), ADJ, ft ? (int)sizeof(TF) : 0, g.ntot);
+  RowsCfg cfg = rows_cfg((int)sizeof(TS), ADJ, ft ? (int)sizeof(TF) : 0, g.ntot, g.n[1]);
   MarchArgs a;
   a.sr_key = sr_key;
   a.n0 = g.n[0];
@@ -1643,7 +1647,7 @@ hipError_t rows_dispatch(const Grid3& g, const TS* in, TS* out, const int dirs[3
   // tile), the fixed array of the allocation-free entry point: many narrow
   // tiles keep the taller shape.
   if (ADJ && ft && a.tiles2 * tiles1() > 16384)
-    cfg = rows_cfg((int)sizeof(TS), ADJ, (int)sizeof(TF), INT64_MAX);
+    cfg = rows_cfg((int)sizeof(TS), ADJ, (int)sizeof(TF), INT64_MAX, a.n1);
   const int R = cfg.R, WY = cfg.WY;
   a.tiles1 = tiles1();
   const int64_t tiles = a.tiles2 * a.tiles1;
@@ -2377,6 +2381,10 @@ int plan_pass(int dtype, const Grid3& g, int left, int cap) {
     }
   }
   return first[left];
+}
+
+int one_step_waves(int dtype, const Grid3& g) {
+  return rows_cfg((int)dtype_size(dtype), false, 0, g.ntot, g.n[1]).WY;
 }
 
 int64_t picked_chunk(int dtype, const Grid3& g, int k, int* rows) {

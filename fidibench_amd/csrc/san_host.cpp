@@ -311,6 +311,20 @@ void long_grid_chunks() {
       }
 }
 
+// Grids of up to four rows a plane take blocks of two waves, of two rows each.
+void one_step_shapes() {
+  const double v[3] = {0.3, -0.2, 0.1}, len[3] = {1, 1, 1};
+  for (int dt : {FDB_F64, FDB_F32, FDB_BF16, FDB_BF16_SR})
+    for (uint64_t n1 : {1, 2, 4, 5, 40}) {
+      const uint64_t n[3] = {7, n1, 900};
+      fdb::Grid3 g, g1;
+      check(fdb::make_grid(3, n, v, len, 1e-3, &g), "grid");
+      check(fdb::one_step_waves(dt, g) == (n1 <= 4 ? 2 : 4), "waves of a step");
+      check(fdb::make_grid(1, n + 2, v, len, 1e-3, &g1), "grid");
+      check(fdb::one_step_waves(dt, g1) == 2, "waves of a 1-D step");
+    }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -334,6 +348,7 @@ int main(int argc, char** argv) {
     one_step_routes(false);
     long_grid_chunks();
     picked_shapes();
+    one_step_shapes();
     plans();
     folds_and_vtk();
     fold_maps();

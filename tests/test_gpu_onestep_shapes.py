@@ -58,3 +58,32 @@ def test_adjoint_step_bit_exact_across_shape_rules(oracle, shape):
         up = 1 if v[j] < 0 else -1
         scale = float(np.abs(lam_next * (np.roll(f, -up, j) - f)).sum())
         assert abs(s[2 * j] + s[2 * j + 1] - terms[j]) <= 1e-11 * scale
+
+
+# Up to four rows a plane: blocks of two waves of two rows.
+FEW_ROWS = [(1,), (63,), (131303,), (5, 1, 130), (3, 2, 65), (40, 3, 257), (9, 4, 1000), (9, 5, 96)]
+
+
+@pytest.mark.parametrize("shape", FEW_ROWS)
+@pytest.mark.parametrize("dtype", ["f64", "f32", "bf16", "bf16sr"])
+def test_one_step_bit_exact_with_few_rows(oracle, shape, dtype):
+    from fidibench_amd import Upwind, configs as K
+    for sign in (1.0, -1.0):
+        v, one = tuple(sign * x for x in (0.3, -0.45, 0.2)[:len(shape)]), (1.0,) * len(shape)
+        dt = K.cfl_dt(shape, v)
+        f0 = oracle.uniform(shape, 0.0, 1.0, seed=sum(shape))
+        with Upwind(v, one, shape, dtype=dtype) as up:
+            up.set_field(f0)
+            start = up.get_field()
+            if dtype == "bf16sr":
+                up.set_seed(5)
+                ref = oracle.advect_bf16_sr(start, v, one, dt, 2, seed=5)
+            else:
+                ref = oracle.advect(start, v, one, dt, 2)
+            up.advect(2, dt)
+            assert np.array_equal(bits(up.get_field()), bits(ref))
+
+
+@pytest.mark.parametrize("shape", [(9, 1, 130), (30, 2, 65), (7, 4, 301), (1, 3, 5000)])
+def test_adjoint_step_bit_exact_with_few_rows(oracle, shape):
+    test_adjoint_step_bit_exact_across_shape_rules(oracle, shape)
