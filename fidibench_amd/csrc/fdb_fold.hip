@@ -46,9 +46,6 @@ constexpr int kFoldTile = kFoldThreads * kFoldPer;        // values staged in LD
 constexpr uint64_t kFoldMaxChunks = 16384;
 constexpr size_t kFoldGatherBytes = 16u << 20;            // chunks copied out, at most
 constexpr double kTwo52 = 4503599627370496.0;
-// Device-side slack around the binade's ends, in units of u: the guessed s
-// is a sum in another order (relative error far below 2^-38).
-constexpr double kGuessSlack = 16384.0;
 
 __device__ inline double fold_ld(const double* x, uint64_t i) { return x[i]; }
 __device__ inline double fold_ld(const float* x, uint64_t i) { return (double)x[i]; }
@@ -187,8 +184,7 @@ __global__ __launch_bounds__(kFoldThreads) void fold_map_kernel(
     rec.neg = neg;
     rec.slot = -1;
     const double m0 = ldexp(fabs(s0), scale);
-    const bool fits = !any_bad && m0 + rec.lo >= kTwo52 + kGuessSlack &&
-                      m0 + rec.hi <= 2.0 * kTwo52 - kGuessSlack;
+    const bool fits = !any_bad && fold_fits(m0, rec.lo, rec.hi, fold_slack(n));
     rec.kind = !any_value ? kFoldZero : (fits ? kFoldMapped : kFoldRaw);
     slot = slots;
     if (rec.kind == kFoldRaw) {

@@ -53,6 +53,22 @@ __host__ __device__ inline void fold_append(FoldMap& m, double v) {
   m.hi = fmax(m.hi, fmax(m.d0, m.d1));
 }
 
+// How far (in u) the loop's s may be from the sum in another order that
+// guesses it: half a unit for each of the loop's n additions, which drift one
+// way where all round alike (2^27 values of 0.1: a relative 2^-28.7), and the
+// other sum's few.  (Where |s| was in a higher binade before, it may be
+// further off: fold_step sees that.)
+__host__ __device__ inline double fold_slack(unsigned long long n) {
+  return 0.5 * (double)n + 16384.0;
+}
+
+// Whether s stays in its binade from the guessed start m0 on, through every
+// value, however the slack falls.
+__host__ __device__ inline bool fold_fits(double m0, double lo, double hi, double slack) {
+  const double first = 4503599627370496.0 + slack, last = 2.0 * 4503599627370496.0 - slack;
+  return m0 >= first && m0 <= last && m0 + lo >= first && m0 + hi <= last;
+}
+
 }  // namespace fdb
 
 #endif

@@ -141,6 +141,42 @@ void fold_maps() {
   check(bad == 0, "fold maps equal the sequential loop");
 }
 
+// The chunks of a field of equal values, mapped where the guessed sum (in
+// another order) lets them: every map must apply to the loop's own sum, which
+// drifts from the guess as all additions round alike.  Values that bring the
+// sum to a power of two at a chunk's start, and next to them.
+void fold_guesses() {
+  const uint64_t chunk = 2048, n = 600 * chunk;
+  int bad = 0, mapped = 0;
+  for (uint64_t at : {3, 77, 300, 599})
+    for (int near = -40; near <= 40; ++near) {
+      double x = std::ldexp(1.0, 3) / (double)(at * chunk);
+      for (int i = 0; i < std::abs(near); ++i) x = std::nextafter(x, near < 0 ? 0.0 : 1.0);
+      double s = 0.0;
+      for (uint64_t c = 0; c * chunk < n; ++c) {
+        const double guess = (double)(c * chunk) * x;
+        const int ex = std::ilogb(guess);
+        double want = s;
+        for (uint64_t i = 0; i < chunk; ++i) want = want + x;
+        if (guess > 0.0) {
+          fdb::FoldMap m = fdb::fold_identity();
+          fdb::fold_append(m, std::ldexp(x, 52 - ex));
+          for (uint64_t k = 1; k < chunk; k *= 2) m = fdb::fold_then(m, m);
+          if (fdb::fold_fits(std::ldexp(guess, 52 - ex), m.lo, m.hi, fdb::fold_slack(n))) {
+            const fdb::FoldRec rec{m.d0, m.d1, m.lo, m.hi, ex, 0, fdb::kFoldMapped, -1};
+            double got = s;
+            ++mapped;
+            if ((!fdb::fold_step(rec, nullptr, chunk, chunk, &got) || got != want) && ++bad <= 4)
+              std::fprintf(stderr, "fold guess: at %d near %d chunk %d s %a guess %a\n", (int)at,
+                           near, (int)c, s, guess);
+          }
+        }
+        s = want;
+      }
+    }
+  check(bad == 0 && mapped > 4 * 81 * 500, "guessed sums hold");
+}
+
 void write_file(const std::string& path, const std::vector<unsigned char>& bytes) {
   FILE* fp = std::fopen(path.c_str(), "wb");
   if (!fp) {
@@ -352,6 +388,7 @@ int main(int argc, char** argv) {
     plans();
     folds_and_vtk();
     fold_maps();
+    fold_guesses();
     raw_headers();
     cli();
     constructors();

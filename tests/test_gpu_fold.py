@@ -121,3 +121,14 @@ def test_values_next_to_a_tie_add_up(oracle):
         with Upwind((1.0,), (1.0,), (g.size,)) as up:
             up.set_field(g)
             assert up.checksum().hex() == oracle.checksum(g).hex()
+
+
+@pytest.mark.parametrize("n", [300 * 2048, 5000000])
+def test_equal_values_drift_from_the_guess(oracle, n):
+    """Sums that reach a power of two at a chunk's start."""
+    from fidibench_amd import Upwind
+    for x in (0.1, 8.0 / (3 * 2048), 8.0 / (77 * 2048), -1.0 / (5 * 2048)):
+        f = np.full(n, x)
+        with Upwind((1.0,), (1.0,), (n,)) as up:
+            up.set_field(f)
+            assert np.float64(up.checksum()).tobytes() == np.float64(oracle.checksum(f)).tobytes()
