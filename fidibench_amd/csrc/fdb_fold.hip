@@ -213,8 +213,12 @@ FoldPlan fold_plan(uint64_t n) {
   const uint64_t per = (n + kFoldMaxChunks - 1) / kFoldMaxChunks;
   p.chunk = std::max<uint64_t>(1, (per + kFoldTile - 1) / kFoldTile) * kFoldTile;
   p.nchunks = (n + p.chunk - 1) / p.chunk;
-  p.slots = std::max<uint64_t>(
-      8, std::min<uint64_t>(p.nchunks / 4 + 16, kFoldGatherBytes / (p.chunk * sizeof(double))));
+  // Chunks that can be copied out: all of them up to kFoldGatherBytes (fields
+  // whose sum keeps passing through zero have no others, and fold on the host
+  // from the copies), else a quarter.
+  const uint64_t most = kFoldGatherBytes / (p.chunk * sizeof(double));
+  p.slots = p.nchunks <= most ? p.nchunks
+                              : std::max<uint64_t>(8, std::min<uint64_t>(p.nchunks / 4 + 16, most));
   // [count | records | copied chunks | prefix sums]
   p.rec_off = 64;
   p.gather_off = (p.rec_off + p.nchunks * sizeof(FoldRec) + 63) / 64 * 64;

@@ -177,6 +177,19 @@ void fold_guesses() {
   check(bad == 0 && mapped > 4 * 81 * 500, "guessed sums hold");
 }
 
+// The fold's plan: every chunk of fields up to 16 MB can be copied out, and
+// what larger ones copy fits the 64 MiB staging buffer.
+void fold_plans() {
+  for (uint64_t n : {65536ull, 65537ull, 400000ull, 2097152ull, 2097153ull, 1ull << 27, 1ull << 33}) {
+    const fdb::FoldPlan p = fdb::fold_plan(n);
+    check(p.nchunks * p.chunk >= n && (p.nchunks - 1) * p.chunk < n && p.nchunks <= 16384, "chunks");
+    check(n * 8 > (16u << 20) || p.slots == p.nchunks, "every chunk has a slot");
+    check(p.slots >= 8 && p.slots <= p.nchunks && p.host_bytes <= (64u << 20) &&
+              p.host_bytes >= p.gather_off + p.slots * p.chunk * 8 && p.dev_bytes > p.host_bytes,
+          "slots");
+  }
+}
+
 void write_file(const std::string& path, const std::vector<unsigned char>& bytes) {
   FILE* fp = std::fopen(path.c_str(), "wb");
   if (!fp) {
@@ -389,6 +402,7 @@ int main(int argc, char** argv) {
     folds_and_vtk();
     fold_maps();
     fold_guesses();
+    fold_plans();
     raw_headers();
     cli();
     constructors();
