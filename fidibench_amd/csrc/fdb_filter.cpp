@@ -6,6 +6,7 @@
 #include <algorithm>
 #include <cstring>
 #include <fstream>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -25,6 +26,7 @@ struct fdb_filter {
   hipEvent_t e0 = nullptr, e1 = nullptr;
   char* fold_dev = nullptr;   // scratch of the exact fold (first checksum on)
   char* fold_host = nullptr;  // its pinned host side
+  std::mutex fold_mutex;      // checksums may come from several threads
 };
 
 namespace {
@@ -237,6 +239,7 @@ int fdb_filter_checksum(fdb_filter_t* h, int which, double* out) {
   // chunk on the host.
   if ((uint64_t)h->g.ntot >= fdb::kFoldMinValues) {
     const fdb::FoldPlan p = fdb::fold_plan((uint64_t)h->g.ntot);
+    std::lock_guard<std::mutex> lock(h->fold_mutex);
     if (!h->fold_dev && hipMalloc((void**)&h->fold_dev, p.dev_bytes) != hipSuccess)
       h->fold_dev = nullptr;
     if (!h->fold_host && hipHostMalloc((void**)&h->fold_host, p.host_bytes) != hipSuccess)

@@ -132,3 +132,30 @@ def test_equal_values_drift_from_the_guess(oracle, n):
         with Upwind((1.0,), (1.0,), (n,)) as up:
             up.set_field(f)
             assert np.float64(up.checksum()).tobytes() == np.float64(oracle.checksum(f)).tobytes()
+
+
+def test_checksums_of_one_filter_from_several_threads(oracle):
+    """Each thread's folds share the filter's scratch."""
+    import threading
+    from fidibench_amd import Filter
+    n = 300 * 2048 + 5
+    f = np.random.default_rng(4).standard_normal(n)
+    flt = Filter((n,), (0.0,), (1.0,), {(0,): 2.0, (1,): -0.5})
+    flt.setInData(f)
+    flt.applyFilter()
+    want = {"input": oracle.checksum(f), "output": oracle.checksum(flt.get_data("output"))}
+    wrong = []
+
+    def fold(which):
+        for _ in range(20):
+            got = flt.computeCheckSum(which)
+            if np.float64(got).tobytes() != np.float64(want[which]).tobytes():
+                wrong.append((which, got))
+
+    threads = [threading.Thread(target=fold, args=(w,)) for w in ("input", "output") * 2]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    flt.close()
+    assert not wrong
