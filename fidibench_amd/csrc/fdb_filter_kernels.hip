@@ -641,6 +641,12 @@ int64_t star_block_tiles(const FilterGeom& g, FilterMarch& m) {
 bool star_block_plan(const FilterGeom& g, int R, bool flat, FilterPlan* p) {
   const int64_t bytes = 16 * g.n[0] * g.n[1] * g.n[2];
   if (!flat && bytes > (R == 1 ? kFilterResident : kStarBlockMax2)) return false;
+  // Planes of eight rows fill the marching kernel's 128 x 8 tiles and half of
+  // the block form's 32 x 16 ones: radius 2, us marching / block, 20000x8x6 9.2
+  // / 12.6, 128x8x2000 10.9 / 13.5, 8000x8x120 32 / 38; below 8 MiB or 128
+  // columns the block form (1000x8x64 6.9 / 6.8, 30x8x30000 68 / 38).  (Nine
+  // rows: 4000x9x150 29 / 26.)
+  if (!flat && R == 2 && g.n[1] <= 8 && g.n[0] >= 128 && bytes > (8ll << 20)) return false;
   if (16 * g.n[0] * 8 >= 0x7fffffffLL) return false;  // store offsets within a tile
   p->stream = bytes > kFilterResident;
   for (bool small : {false, true}) {

@@ -374,6 +374,24 @@ void one_step_shapes() {
     }
 }
 
+// Star stencils over planes of eight rows: the block form where the grid is
+// small or narrow, the marching kernel otherwise.
+void filter_routes() {
+  auto block = [](int64_t n0, int64_t n1, int64_t n2, int R) {
+    fdb::FilterGeom g{};
+    g.n[0] = n0, g.n[1] = n1, g.n[2] = n2;
+    const int order[5] = {0, 1, 2, 1, 0}, lo[5] = {-R, -R, -R, 1, 1}, hi[5] = {-1, -1, R, R, R};
+    for (int b = 0; b < 5; ++b)
+      for (int k = lo[b]; k <= hi[b]; ++k) g.off[g.nt++][order[b]] = k;
+    fdb::FilterPlan p{};
+    check(fdb::plan_filter(g, &p) == hipSuccess, "filter plan");
+    return p.block;
+  };
+  check(!block(20000, 8, 6, 2) && !block(128, 8, 2000, 2) && !block(2000, 8, 64, 2), "marching");
+  check(block(20000, 8, 6, 1) && block(1000, 8, 64, 2) && block(30, 8, 30000, 2) &&
+            block(4000, 9, 150, 2) && block(100, 8, 7, 2), "blocks");
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -398,6 +416,7 @@ int main(int argc, char** argv) {
     long_grid_chunks();
     picked_shapes();
     one_step_shapes();
+    filter_routes();
     plans();
     folds_and_vtk();
     fold_maps();

@@ -63,3 +63,11 @@ def test_kernel_choice_by_size_bit_exact_vs_oracle(oracle, dims, R):
     ref = oracle.filter_apply(f0, dims, list(st.items()))
     assert np.array_equal(bits(flt.get_data("output").ravel(order="F")), bits(ref))
     flt.close()
+
+
+# Planes of eight rows, radius 2: marched from 8 MiB (16 bytes a cell) and 128
+# columns on, in blocks below.
+@pytest.mark.parametrize("dims", [(127, 8, 530), (128, 8, 512), (128, 8, 513), (2000, 8, 33),
+                                  (2001, 8, 40), (20000, 8, 6)])
+def test_planes_of_eight_rows_bit_exact_vs_oracle(oracle, dims):
+    test_block_kernel_bit_exact_vs_oracle(oracle, dims, 2)
