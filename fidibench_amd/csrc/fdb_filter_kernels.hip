@@ -254,9 +254,9 @@ __global__ __launch_bounds__(256) void filter_march_kernel(const double* __restr
 // are unconditional, as in the ring kernel.  Stores go past the caches (NT)
 // only where the fields exceed the Infinity Cache: 256^3 58.3 -> 50.5 us
 // cached, 512^3 416 -> 432.
-template <int R_, int BX, int CX, int CY>
+template <int R>
 struct StarShape {
-  static constexpr int R = R_, kBX = BX, kBY = 256 / BX, kCX = CX, kCY = CY;
+  static constexpr int kBX = 64, kBY = 4, kCX = 2, kCY = 2;
   static constexpr int kTX = kBX * kCX, kTY = kBY * kCY;
   static constexpr int kLX = kTX + 2 * R, kLY = kTY + 2 * R, kNE = kLX * kLY;
   static constexpr int kNH = kNE - kTX * kTY;    // halo-ring values per plane
@@ -264,11 +264,11 @@ struct StarShape {
   static constexpr size_t kLds = 2 * (kNE + 64) * sizeof(double);
 };
 
-template <class S, bool NT>
+template <int R, bool NT>
 __global__ __launch_bounds__(256) void filter_star_kernel(const double* __restrict__ in,
                                                           double* __restrict__ out,
                                                           FilterGeom g, FilterMarch m) {
-  constexpr int R = S::R;
+  using S = StarShape<R>;
   constexpr int BX = S::kBX, BY = S::kBY, CX = S::kCX, CY = S::kCY;
   constexpr int LX = S::kLX, NE = S::kNE, NH = S::kNH, NLH = S::kNLH, D = 2 * R + 1;
   static_assert(R == 1 || R == 2, "the plane loop is unrolled for 4 or 6 queue slots");
@@ -599,25 +599,28 @@ constexpr int64_t kStarBlockMax2 = 160ll << 20;
 constexpr int64_t kSmallStarBlocks = 256;
 
 // Calls f(S{}, kernel) for the block form of radius R (FLAT: 2-D).  small:
-// fewer planes per block, for grids with less than a block per CU.
+// fewer planes per block, for grids with less than a block per CU.  stream:
+// stores past the caches, which only large 2-D fields take (3-D ones that large
+// march, small blocks are of small fields).
 template <class F>
 hipError_t with_star_block(int R, bool flat, bool small, bool stream, F f) {
-#define FDB_SB(R, BX, CY, C, FL, BA)                                          \
-  do {                                                                        \
-    using S = StarBlock<R, BX, 1, CY, C, FL, BA>;                             \
-    return stream ? f(S{}, &filter_star_block_kernel<S, true>)                \
-                  : f(S{}, &filter_star_block_kernel<S, false>);              \
+#define FDB_SB(R, BX, CY, C, FL, BA, NT)                   \
+  do {                                                     \
+    using S = StarBlock<R, BX, 1, CY, C, FL, BA>;          \
+    return f(S{}, &filter_star_block_kernel<S, NT>);       \
   } while (0)
   if (flat) {
-    if (R == 1 && small) FDB_SB(1, 256, 1, 4, true, true);
-    if (R == 1) FDB_SB(1, 256, 1, 8, true, true);
-    if (small) FDB_SB(2, 256, 1, 4, true, true);
-    FDB_SB(2, 256, 1, 8, true, true);
+    if (R == 1 && small) FDB_SB(1, 256, 1, 4, true, true, false);
+    if (R == 1 && stream) FDB_SB(1, 256, 1, 8, true, true, true);
+    if (R == 1) FDB_SB(1, 256, 1, 8, true, true, false);
+    if (small) FDB_SB(2, 256, 1, 4, true, true, false);
+    if (stream) FDB_SB(2, 256, 1, 8, true, true, true);
+    FDB_SB(2, 256, 1, 8, true, true, false);
   }
-  if (R == 1 && small) FDB_SB(1, 32, 1, 2, false, true);
-  if (R == 1) FDB_SB(1, 32, 2, 4, false, false);
-  if (small) FDB_SB(2, 32, 1, 2, false, true);
-  FDB_SB(2, 32, 2, 4, false, false);
+  if (R == 1 && small) FDB_SB(1, 32, 1, 2, false, true, false);
+  if (R == 1) FDB_SB(1, 32, 2, 4, false, false, false);
+  if (small) FDB_SB(2, 32, 1, 2, false, true, false);
+  FDB_SB(2, 32, 2, 4, false, false, false);
 #undef FDB_SB
 }
 
@@ -676,7 +679,7 @@ hipError_t launch_star_block(const FilterPlan& p, const double* in, double* out,
 
 template <int R>
 bool star_plan(const FilterGeom& g, FilterMarch& m, int64_t& blocks) {
-  using S = StarShape<R, 64, 2, 2>;
+  using S = StarShape<R>;
   m = FilterMarch{};
   m.rx = m.ry = m.rz = R;
   m.LX = S::kLX;
@@ -689,7 +692,7 @@ bool star_plan(const FilterGeom& g, FilterMarch& m, int64_t& blocks) {
   m.tiles_y = (g.n[1] + S::kTY - 1) / S::kTY;
   const int64_t tiles = m.tiles_x * m.tiles_y;
   const int64_t cap =
-      kernel_capacity(reinterpret_cast<const void*>(&filter_star_kernel<StarShape<R, 64, 2, 2>, true>), 256, 0);
+      kernel_capacity(reinterpret_cast<const void*>(&filter_star_kernel<R, true>), 256, 0);
   const int64_t per_round = std::max<int64_t>(1, cap / tiles);
   const int64_t nch = march_chunks(tiles, g.n[2], 2 * R, cap,
                                    std::max<int64_t>(1, per_round / 2), 4 * per_round, true);
@@ -889,8 +892,7 @@ hipError_t launch_filter(const FilterPlan& p, const double* in, double* out, hip
   if (p.kind == kFilterPlanesWide) return launch_march<March3DWide>(p, in, out, s);
   if (p.kind == kFilterStar) {
     const dim3 grid((unsigned)p.blocks), block(64, 4);
-    auto* kern = p.stream ? &filter_star_kernel<StarShape<2, 64, 2, 2>, true>
-                          : &filter_star_kernel<StarShape<2, 64, 2, 2>, false>;
+    auto* kern = p.stream ? &filter_star_kernel<2, true> : &filter_star_kernel<2, false>;
     hipLaunchKernelGGL(kern, grid, block, 0, s, in, out, p.g, p.m);
     return hipGetLastError();
   }
