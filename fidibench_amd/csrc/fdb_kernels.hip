@@ -15,7 +15,6 @@
 
 #include <cmath>
 #include <mutex>
-#include <vector>
 
 #include "fdb_internal.h"
 #include "../../include/fidibench_amd/fdb_upwind.h"
@@ -1719,9 +1718,6 @@ hipError_t rows_dispatch(const Grid3& g, const TS* in, TS* out, const int dirs[3
 // x 4 waves at K <= 4 (tb_default; FDB_TB_CFG_<bytes>_<K> overrides).
 TbCfg tb_cfg(int bytes, int K) { return tuning().tb[bytes][K]; }
 
-// levels != nullptr: also store levels 1..K-1 to levels[0..K-2] (K = 4
-// or 8, FP64 only: with one 4-byte cell per lane the FP32 kernel writes its
-// 8 levels at ~2 TB/s, slower than one-step launches storing 16 B per lane).
 // Launch shape of the stochastic-rounding bf16 pass (K = 2, 4 or 8): an
 // even number of rows per wave and an even K, so the wave's rows start at
 // an even row and hold whole pairs; within 128 VGPRs, i.e. four waves per
@@ -1939,6 +1935,10 @@ bool small_store_all(int bytes, const Grid3& g, int K) {
          g.ntot < (bytes == 8 ? kStoreAllCells64 : kStoreAllCells32);
 }
 
+// levels != nullptr: also store levels 1..K-1 to levels[0..K-2]: FP64 with K = 4
+// or 8, FP32 with K = 4 below kStoreAllCells32 cells (at 512^3 it writes the
+// levels slower than one-step launches storing 16 B per lane), never 2-byte
+// storage.
 // visits != nullptr: launch nothing; store the pass's length in row-plane
 // visits of one resident block slot instead (rounds of resident blocks x
 // planes per block, warm-up planes included, x rows per wave), from the same
@@ -2478,21 +2478,31 @@ hipError_t launch_advect_pass(int dtype, const Grid3& g, void* const bufs[2], in
 hipError_t launch_planned_steps(int dtype, const Grid3& g, const void* src, void* dst, void* tmp,
                                 int nsteps, int cap, hipStream_t s, uint64_t step0,
                                 uint64_t seed) {
-  std::vector<int> ks;
-  for (int left = nsteps; left > 0; left -= ks.back())
-    ks.push_back(plan_pass(dtype, g, left, cap));
+  // Passes in all: the last one lands in dst.  (No list of them: nothing here
+  // allocates, so nothing throws into a C caller.  Above kPlanTail steps every
+  // pass is the same.)
+  int64_t passes = 0;
+  int left = nsteps;
+  if (left > kPlanTail) {
+    const int k = plan_pass(dtype, g, left, cap);
+    passes = (left - kPlanTail + k - 1) / k;
+    left -= (int)passes * k;
+  }
+  for (; left > 0; ++passes) left -= plan_pass(dtype, g, left, cap);
   const void* from = src;
-  for (size_t i = 0; i < ks.size(); ++i) {
-    void* to = (ks.size() - 1 - i) % 2 == 0 ? dst : tmp;  // the last one lands in dst
+  for (left = nsteps; left > 0;) {
+    void* to = --passes % 2 == 0 ? dst : tmp;
     if (!to || to == from) return hipErrorInvalidValue;
     void* const pair[2] = {const_cast<void*>(from), to};
     int cur = 0;
+    const int k = plan_pass(dtype, g, left, cap);
     const hipError_t err =
-        ks[i] > 1 ? launch_fused_pass(dtype, g, from, to, ks[i], s, nullptr, step0, seed)
-                  : launch_advect_pass(dtype, g, pair, &cur, 1, s, nullptr, step0, seed);
+        k > 1 ? launch_fused_pass(dtype, g, from, to, k, s, nullptr, step0, seed)
+              : launch_advect_pass(dtype, g, pair, &cur, 1, s, nullptr, step0, seed);
     if (err != hipSuccess) return err;
     from = to;
-    step0 += (uint64_t)ks[i];
+    left -= k;
+    step0 += (uint64_t)k;
   }
   return hipSuccess;
 }

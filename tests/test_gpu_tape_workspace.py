@@ -118,6 +118,13 @@ def test_advect_from_equals_advect(dtype, shape, n):
                                        s) == L.ERR_INVALID
 
 
+@pytest.mark.parametrize("n", [47, 48, 49, 55, 97, 150])
+def test_advect_from_of_long_runs(n):
+    """Runs past those the planner splits exactly, odd and even pass counts."""
+    for dtype, shape in (("f64", SHAPE), ("f32", (30, 70)), ("bf16sr", SHAPE), ("bf16", (41,))):
+        test_advect_from_equals_advect(dtype, shape, n)
+
+
 def test_forward_without_gradient_keeps_its_input_and_takes_strided_fields():
     from fidibench_amd import autograd as A
     big = torch.rand((12, 40, 200), device="cuda", dtype=torch.float64)
