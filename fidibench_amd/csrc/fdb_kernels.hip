@@ -2182,7 +2182,9 @@ bool make_grid(int ndims, const uint64_t* n, const double* v, const double* len,
   return true;
 }
 
-float rows_step_us(int dtype, const Grid3& g) {
+namespace {
+// Time (us) of the row tiles a step by the rows kernel issues.
+double rows_issue_us(int dtype, const Grid3& g) {
   const int bytes = (int)dtype_size(dtype);
   int vec = 16 / bytes;
   while (vec > 1 && g.n[2] % vec != 0) vec >>= 1;
@@ -2192,9 +2194,14 @@ float rows_step_us(int dtype, const Grid3& g) {
   static constexpr double k64[2] = {0.115, 0.033}, k32[2] = {0.013, 0.074},
                           k16[2] = {0.045, 0.046}, ksr[2] = {0.033, 0.068};
   const double* k = bytes == 8 ? k64 : (bytes == 4 ? k32 : (dtype == FDB_BF16_SR ? ksr : k16));
-  const double moved = 2.0 * (double)g.ntot * bytes;
+  return 1e-3 * tiles * (k[0] + k[1] * vec);
+}
+}  // namespace
+
+float rows_step_us(int dtype, const Grid3& g) {
+  const double moved = 2.0 * (double)g.ntot * (double)dtype_size(dtype);
   const double mem = moved / (moved <= (double)kResidentBytes ? 6.6e6 : 5.2e6);
-  return (float)(3.6 + std::max(mem, 1e-3 * tiles * (k[0] + k[1] * vec)));
+  return (float)(3.6 + std::max(mem, rows_issue_us(dtype, g)));
 }
 
 bool fused_pass_supported(int dtype, const Grid3& g, int k) {
@@ -2256,11 +2263,13 @@ int64_t fused_pass_visits(int dtype, const Grid3& g, int k) {
 
 // Launch times (us) of every depth over g (0: no such pass).  On grids of at
 // least 512^3 cells the 512^3 times are scaled to g: the one-step kernel by
-// the cell count, a fused pass by its length in plane visits (its blocks take
-// equal time per plane there, so the length captures rounds of resident
-// blocks, warm-up planes and tiles cut by the grid's extents; at 1024^3 FP64
-// this picks 8-step passes, 679 us per step, over 7-step ones, 710).  On
-// smaller grids the pass's own model (pick_pass, sr_pass_us).
+// the cell count (or by the rows it issues, where these are short: 20000 x 90
+// x 100 bf16 271 us a step, 134 by its cells), a fused pass by its length in
+// plane visits (its blocks take equal time per plane there, so the length
+// captures rounds of resident blocks, warm-up planes and tiles cut by the
+// grid's extents; at 1024^3 FP64 this picks 8-step passes, 679 us per step,
+// over 7-step ones, 710).  On smaller grids the pass's own model (pick_pass,
+// sr_pass_us).
 struct PassCosts {
   float us[kMaxTimeBlock + 1];
 };
@@ -2306,7 +2315,7 @@ PassCosts pass_costs(int dtype, const Grid3& g) {
     return c;
   }
   const int64_t* ref = ref_visits() + row * (kMaxTimeBlock + 1);
-  c.us[1] = tab[1] * (float)cells;
+  c.us[1] = std::max(tab[1] * (float)cells, (float)rows_issue_us(dtype, g));
   for (int k = 2; k <= kMaxTimeBlock; ++k) {
     if (tab[k] <= 0.0f || ref[k] <= 0 || !fused_pass_supported(dtype, g, k)) continue;
     const int64_t v = fused_pass_visits(dtype, g, k);

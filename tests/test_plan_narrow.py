@@ -21,6 +21,8 @@ def _passes(dtype, shape, nsteps=22):
     ("BF16", (400, 400, 16)),   # 16.7 / 4.1
     ("BF16", (300507, 14)),     # 62 / 9
     ("F32", (2077634, 3)),      # 243 / 44
+    ("BF16", (3000, 3000, 16)),  # 790 / 172, above 512^3 cells
+    ("F64", (5000, 9000, 4)),   # 5259 / 1229
 ])
 def test_short_rows_take_several_steps_a_launch(dtype, shape):
     assert 1 not in _passes(dtype, shape)
