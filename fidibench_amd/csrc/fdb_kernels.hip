@@ -851,6 +851,7 @@ struct TbArgs {
 
 // Modes of the temporally blocked kernel.
 //   kTbPlain     K forward steps, level K stored to out.
+//   kTbStream    the same with its stores past the caches (see kStream)
 //   kTbStoreAll  also levels 1..K-1 stored, to aux.lv[0..K-2] (a forward
 //                that keeps every state).
 //   kTbAdjoint   the fused transpose (adjoint) pass.  The kernel is called
@@ -874,7 +875,7 @@ struct TbArgs {
 //                lane holds both rows of each of its pairs (even rows per
 //                wave, even K, even n1), so each lane hashes one word per
 //                pair of rows and level, with no exchange between lanes.
-constexpr int kTbPlain = 0, kTbStoreAll = 1, kTbAdjoint = 2, kTbSR = 3, kTbAdjLast = 4;
+constexpr int kTbPlain = 0, kTbStoreAll = 1, kTbAdjoint = 2, kTbSR = 3, kTbAdjLast = 4, kTbStream = 5;
 struct TbAux {
   const void* fs[kMaxTimeBlock];
   void* lv[kMaxTimeBlock];
@@ -1020,7 +1021,8 @@ __global__ __launch_bounds__(64 * WY) void tb_kernel(const TS* __restrict__ in,
   // shape keeps one plane per trip within 128 VGPRs.)
   constexpr bool kTwoPlanes = !PROD && (K <= 6 || (sizeof(M) == 8 && R * K == 56));
   constexpr bool kCondPrefetch = PIPE && !kTwoPlanes;
-  constexpr bool kWaitBeforeStores = (MODE == kTbPlain || MODE == kTbSR) && !kCondPrefetch;
+  constexpr bool kWaitBeforeStores =
+      (MODE == kTbPlain || MODE == kTbSR || MODE == kTbStream) && !kCondPrefetch;
   // The result's stores.  A tile's rows end inside cache lines that the
   // neighbouring tile, on the same XCD at about the same time, completes:
   // through the caches the halves meet in L2, and the next pass finds the
@@ -1031,8 +1033,10 @@ __global__ __launch_bounds__(64 * WY) void tb_kernel(const TS* __restrict__ in,
   // 380 / 352; FP64 4 rows K = 6 at 256^3 14.6 / 13.5.  The FP64 shapes of
   // large grids lose (K = 7 512^3 91.7 / 93.1, 1024 x 1024 x 768 559 / 605,
   // K = 8 768^3 270 / 277) and stream, as do the two-row shapes, whose
-  // grids stay in the L2s (96^3 10.4 / 10.6 us a pass).
-  constexpr bool kStream = R == 2 || (sizeof(TS) == 8 && R >= 7 && WY == 8);
+  // grids stay in the L2s (96^3 10.4 / 10.6 us a pass).  FP64 9 rows K = 4
+  // does either, by size: 192x200x210 46 / 42 us a pass, 512^3 533 / 563.
+  constexpr bool kStream =
+      R == 2 || MODE == kTbStream || (sizeof(TS) == 8 && R >= 7 && WY == 8);
   // PROD: fv[l] holds the state of level l at the current plane (LASTP:
   // fv[0], the last level's); after its level it is reloaded with the next
   // plane's (always a valid plane, so every load is unconditional).  The
@@ -1986,7 +1990,9 @@ hipError_t tb_dispatch(const Grid3& g, const TS* in, TS* out, int K, hipStream_t
   if (all && sizeof(TS) < 4) return hipErrorNotSupported;
   for (int l = 0; all && l + 1 < K; ++l) aux.lv[l] = levels[l];
   for (int l = 0; sr && l < K; ++l) a.sr_key[l] = sr_fold(sr_keys[l]);
-  const int mode = all ? kTbStoreAll : (sr ? kTbSR : kTbPlain);
+  const bool past = sizeof(TS) == 8 && R == 9 && K == 4 && WY == 4 &&
+                    2 * g.ntot * (int64_t)sizeof(TS) > kResidentBytes;
+  const int mode = all ? kTbStoreAll : (sr ? kTbSR : (past ? kTbStream : kTbPlain));
   bool launched = false;
 #define FDB_TB_DIR(RR, KK, W, L1, L2, MD)                                                   \
   if (!launched && R == RR && K == KK && WY == W && lo1 == L1 && lo2 == L2 &&               \
@@ -2032,6 +2038,7 @@ hipError_t tb_dispatch(const Grid3& g, const TS* in, TS* out, int K, hipStream_t
     FDB_TB(4, 6, 8, kTbPlain)
     FDB_TB(8, 7, 8, kTbPlain)
     FDB_TB(7, 8, 8, kTbPlain)
+    FDB_TB(9, 4, 4, kTbStream)
     FDB_TB(9, 4, 4, kTbStoreAll)
     FDB_TB(9, 8, 8, kTbStoreAll)
     FDB_TB(4, 4, 8, kTbStoreAll)

@@ -229,3 +229,18 @@ def test_time_blocked_bf16_sr_bit_exact(oracle, shape, signs):
         if k >= 2 and shape[1] % 2 == 0 and shape[1] > k:
             assert launches + launches2 < 11  # fused passes ran
         up.close()
+
+
+@pytest.mark.parametrize("shape", [(40, 1000, 430), (30, 1000, 430)])
+def test_four_step_fp64_pass_on_both_sides_of_the_caches(shape):
+    """Its stores go past the caches where both fields exceed 256 MiB."""
+    from fidibench_amd import Upwind
+    for v in ((0.4, -0.3, 0.2), (0.4, 0.3, -0.2), (-0.4, 0.3, 0.2), (-0.4, -0.3, -0.2)):
+        out = []
+        for k in (1, 4):
+            with Upwind(v, (1, 1, 1), shape) as up:
+                up.init_field(1, (0.5, 0.5, 0.5, 0.25, 0.01), seed=4)
+                up.set_time_block(k)
+                up.advect(4, 1e-4)
+                out.append(up.get_field())
+        assert np.array_equal(bits(out[0]), bits(out[1])), v
