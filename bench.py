@@ -406,6 +406,7 @@ def laplacian(iters=10, with_cpu=True):
                               "traffic": pmc_traffic(name,
                                                      "filter_march_kernel_laplacian_stats.md"),
                               "kernel": {"star": "filter_star_kernel (3-D star stencil)",
+                                         # (the 2-D Laplacians: other 2-D stencils march)
                                          "rows": "filter_star_block_kernel (2-D star stencil)"}.get(
                                              flt.kernel(),
                                              f"filter_march_kernel ({flt.kernel()}, 3-D)"),

@@ -89,8 +89,10 @@ class Filter:
 
     # -- extensions --------------------------------------------------------
     def kernel(self) -> str:
-        """The kernel applyFilter launches ("star", "planes", "planes_mid",
-        "planes_wide", "rows" or "gather"; fixed at creation)."""
+        """The family of the kernel applyFilter launches ("star", "planes",
+        "planes_mid", "planes_wide", "rows" or "gather"; fixed at creation).
+        Star stencils under "star", "planes" and "rows" run in blocks with all
+        loads in flight, not marched, where that is faster."""
         name = C.c_char_p()
         L.check(L.lib().fdb_filter_kernel(self._h, C.byref(name)))
         return name.value.decode()

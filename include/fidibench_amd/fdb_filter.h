@@ -53,16 +53,19 @@ int fdb_filter_copy_out_to_in(fdb_filter_t* h);
  * laplacian.cxx:80-86 -- with the kernels' time (HIP events) in *ms. */
 int fdb_filter_iterate_timed(fdb_filter_t* h, int niters, float* ms);
 
-/* The kernel this filter's applyFilter launches, fixed at creation:
+/* The family of the kernel this filter's applyFilter launches, by stencil and
+ * grid, fixed at creation:
  * "star" (full 3-D star stencils of radius 2: the 4th-order
  * Laplacian), "planes", "planes_mid", "planes_wide" (3-D LDS rings),
  * "rows" (2-D) or "gather".  Star stencils named "star", "planes" or "rows"
- * run in blocks with all loads in flight where that is faster.  Extension (no counterpart in the reference). */
+ * run in blocks with all loads in flight, not marched, where that is faster.
+ * Extension (no counterpart in the reference). */
 int fdb_filter_kernel(const fdb_filter_t* h, const char** name);
 
 /* computeCheckSum("input" | "output"), Filter.cpp:466-485: which = 0 for
  * input, 1 for output; the sequential left fold, bit for bit, on the device where
- * the field has 65536 values or more, else on the host. */
+ * the field has 65536 values or more, else on the host.  May be called by several
+ * threads at once. */
 int fdb_filter_checksum(fdb_filter_t* h, int which, double* out);
 
 /* Copies input (which = 0) or output (1) to a host array. */

@@ -232,7 +232,9 @@ int fdb_misfit_dev(int f_dtype, const void* f, const void* target, uint64_t n, i
  * takes lam_T = dL/df_T and returns lam_0 = dL/df0 and dL/dv (host,
  * ndims doubles), recomputing the states it did not keep.  Checkpoints
  * follow the optimal binomial schedule (Griewank's revolve) for the
- * number of field copies that fit in max_bytes of device memory.
+ * number of field copies that fit in max_bytes of device memory; the partial
+ * sums of the velocity products (1 MiB, or what one launch writes) and the
+ * workspace's alignment come on top.
  * f_dtype is the forward storage type, lam_dtype (FDB_F64, FDB_F32 or
  * FDB_BF16) the adjoint's.  All device buffers are caller-owned; both
  * calls block. */
