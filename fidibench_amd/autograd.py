@@ -72,6 +72,7 @@ class Tape:
         if method == "checkpoint" and need.value > _WORKSPACE_MAX:
             self.close()
             h = C.c_void_p()
+            torch.cuda.empty_cache()  # what default_budget counted on
             L.check(L.lib().fdb_tape_create(*args, C.byref(h)))
             self._h = h
             return
@@ -131,8 +132,17 @@ class Tape:
 
 
 def default_budget(fraction: float = 0.85) -> int:
+    """A fraction of the device memory that a checkpointed tape may take: what
+    is free, and what torch's cache holds unused (a tape that allocates its own
+    states has that given back first)."""
     free, _ = torch.cuda.mem_get_info()
-    return int(free * fraction)
+    try:
+        s = torch.cuda.memory_stats()
+    except RuntimeError:  # an allocator without statistics
+        s = {}
+    reserved, active, split = (s.get(f"{k}_bytes.all.current", 0)
+                               for k in ("reserved", "active", "inactive_split"))
+    return int((free + max(0, reserved - active - split)) * fraction)
 
 
 class UpwindAdvect(torch.autograd.Function):
@@ -153,7 +163,12 @@ class UpwindAdvect(torch.autograd.Function):
                                                 int(nsteps), _stream()))
             ctx.tape = None
             return fT
-        budget = max_bytes if max_bytes is not None else default_budget()
+        if max_bytes is not None:
+            budget = max_bytes
+        elif method == "checkpoint" and nsteps * f0c.numel() * f0c.element_size() > _WORKSPACE_MAX:
+            budget = default_budget()
+        else:  # room for every state, or none needed: no statistics to gather
+            budget = int(0.85 * torch.cuda.mem_get_info()[0])
         tape = Tape(f0c.shape, v, lengths, dt, nsteps, f_dtype, lam, budget, method=method)
         fT = torch.empty_like(f0c)
         tape.forward(f0c, fT)

@@ -190,3 +190,24 @@ def _need(shape, T, method):
                                        C.byref(need)))
     L.lib().fdb_tape_destroy(h)
     return need.value
+
+
+def test_budget_counts_torchs_unused_cache_and_a_large_tape_gets_it(monkeypatch):
+    from fidibench_amd import autograd as A
+    torch.cuda.empty_cache()
+    before = A.default_budget(1.0)
+    t = torch.empty(3 << 30, dtype=torch.uint8, device="cuda")
+    assert A.default_budget(1.0) <= before - (2 << 30)
+    del t
+    assert torch.cuda.memory_reserved() >= 3 << 30
+    assert A.default_budget(1.0) >= before - (64 << 20)
+    monkeypatch.setattr(A, "_WORKSPACE_MAX", 1 << 20)
+    f0 = torch.rand(SHAPE, device="cuda", dtype=torch.float64, requires_grad=True)
+    v = torch.tensor(V, dtype=torch.float64)
+    y = A.advect(f0, v, DT, 40, method="checkpoint")
+    assert torch.cuda.memory_reserved() < 1 << 30
+    y.sum().backward()
+    g = f0.grad.clone()
+    f0.grad = None
+    A.advect(f0, v, DT, 40, method="shift").sum().backward()
+    assert torch.equal(g, f0.grad)
