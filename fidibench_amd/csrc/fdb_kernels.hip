@@ -876,6 +876,13 @@ struct TbArgs {
 //                wave, even K, even n1), so each lane hashes one word per
 //                pair of rows and level, with no exchange between lanes.
 constexpr int kTbPlain = 0, kTbStoreAll = 1, kTbAdjoint = 2, kTbSR = 3, kTbAdjLast = 4, kTbStream = 5;
+// Waves per SIMD that a block's registers must leave room for: one block, but
+// two of FP32's transpose pass with products.  Left alone, two of its four
+// sign branches take 130 and 132 VGPRs, hence one block per CU: 1024x1024x768
+// over bf16 states 5870 us a pass against 4820 for the others.
+constexpr int tb_waves(int mode, size_t bytes, int wy) {
+  return mode == kTbAdjoint && bytes == 4 ? 4 : wy / 4;
+}
 struct TbAux {
   const void* fs[kMaxTimeBlock];
   void* lv[kMaxTimeBlock];
@@ -922,9 +929,9 @@ __device__ inline int64_t pmod(int64_t x, int64_t n) {
 
 template <typename TS, int R, int K, int WY, bool LO1, bool LO2, int MODE = kTbPlain,
           typename TF = TS>
-__global__ __launch_bounds__(64 * WY) void tb_kernel(const TS* __restrict__ in,
-                                                     TS* __restrict__ out, TbArgs a,
-                                                     Coef<typename St<TS>::M> cf, TbAux adj) {
+__global__ __launch_bounds__(64 * WY, tb_waves(MODE, sizeof(TS), WY)) void tb_kernel(
+    const TS* __restrict__ in, TS* __restrict__ out, TbArgs a, Coef<typename St<TS>::M> cf,
+    TbAux adj) {
   using M = typename St<TS>::M;
   constexpr bool ALL = MODE == kTbStoreAll, SR = MODE == kTbSR, LASTP = MODE == kTbAdjLast;
   // PROD: velocity products (at every level, or at the last one only);
