@@ -2039,7 +2039,7 @@ hipError_t tb_dispatch(const Grid3& g, const TS* in, TS* out, int K, hipStream_t
   FDB_TB(2, 3, 8, kTbPlain)
   FDB_TB(2, 4, 8, kTbPlain)
   FDB_TB(8, 6, 8, kTbPlain)
-  if constexpr (sizeof(TS) == 4 || sizeof(TS) == 2) FDB_TB(6, 4, 8, kTbPlain)
+  if constexpr (sizeof(TS) < 8) { FDB_TB(6, 4, 8, kTbPlain) }
   if constexpr (sizeof(TS) == 8) {
     FDB_TB(4, 4, 8, kTbPlain)
     FDB_TB(4, 6, 8, kTbPlain)
@@ -2050,7 +2050,7 @@ hipError_t tb_dispatch(const Grid3& g, const TS* in, TS* out, int K, hipStream_t
     FDB_TB(9, 8, 8, kTbStoreAll)
     FDB_TB(4, 4, 8, kTbStoreAll)
   }
-  if constexpr (sizeof(TS) == 4) FDB_TB(6, 4, 8, kTbStoreAll)
+  if constexpr (sizeof(TS) == 4) { FDB_TB(6, 4, 8, kTbStoreAll) }
   if constexpr (sizeof(TS) == 2) {
     FDB_TB(8, 2, 4, kTbSR)
     FDB_TB(8, 4, 4, kTbSR)
