@@ -877,9 +877,10 @@ struct TbArgs {
 //                pair of rows and level, with no exchange between lanes.
 constexpr int kTbPlain = 0, kTbStoreAll = 1, kTbAdjoint = 2, kTbSR = 3, kTbAdjLast = 4, kTbStream = 5;
 // Waves per SIMD that a block's registers must leave room for: one block, but
-// two of FP32's transpose pass with products.  Left alone, two of its four
-// sign branches take 130 and 132 VGPRs, hence one block per CU: 1024x1024x768
-// over bf16 states 5870 us a pass against 4820 for the others.
+// two of FP32's transpose pass with products.  (Two of its four sign branches
+// took 130 and 132 VGPRs, hence one block per CU, with the states loaded by
+// per-lane addresses: 1024x1024x768 over bf16 states 5870 us a pass.  Kept to
+// 128 they spilled 4: 4730.  With the loads by row resources none does: 4600.)
 constexpr int tb_waves(int mode, size_t bytes, int wy) {
   return mode == kTbAdjoint && bytes == 4 ? 4 : wy / 4;
 }
@@ -1052,11 +1053,12 @@ __global__ __launch_bounds__(64 * WY, tb_waves(MODE, sizeof(TS), WY)) void tb_ke
   // anyway), so the states cost no halo traffic.
   M fv[NF][R];
   VAcc acc;
-  uint32_t colf = col;
+  uint32_t cbf = 0;                                       // byte offset of that column
+  const int fbytes = (int)(a.n2 * (int64_t)sizeof(TF));  // row length (TF is no wider than TS)
   int64_t rofff[PROD ? R : 1];
   if constexpr (PROD) {
     const int64_t c_hi = (o2 + 63 - K < a.n2 - 1) ? o2 + 63 - K : a.n2 - 1;
-    colf = (uint32_t)(cl < o2 ? o2 : (cl > c_hi ? c_hi : cl));
+    cbf = (uint32_t)(cl < o2 ? o2 : (cl > c_hi ? c_hi : cl)) * (uint32_t)sizeof(TF);
     const int64_t r_hi = (o1 + WY * R - K - 1 < a.n1 - 1) ? o1 + WY * R - K - 1 : a.n1 - 1;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -1067,7 +1069,7 @@ __global__ __launch_bounds__(64 * WY, tb_waves(MODE, sizeof(TS), WY)) void tb_ke
     for (int l = 0; l < NF; ++l) {
       const TF* fb = (const TF*)adj.fs[l] + pw * plane;
 #pragma unroll
-      for (int r = 0; r < R; ++r) fv[l][r] = (M)St<TF>::ld((fb + rofff[r])[colf]);
+      for (int r = 0; r < R; ++r) fv[l][r] = (M)St<TF>::ld(buf_ld(row_rsrc(fb + rofff[r], fbytes), cbf, fb));
     }
   }
   // One plane, all K levels; each level in place: row r from level l to
@@ -1172,7 +1174,7 @@ __global__ __launch_bounds__(64 * WY, tb_waves(MODE, sizeof(TS), WY)) void tb_ke
           if (l + 1 == K) {  // f_0 at the next plane's output cells
             const TF* fb = (const TF*)adj.fs[0] + pn * plane;
 #pragma unroll
-            for (int r = 0; r < R; ++r) fv[0][r] = (M)St<TF>::ld((fb + rofff[r])[colf]);
+            for (int r = 0; r < R; ++r) fv[0][r] = (M)St<TF>::ld(buf_ld(row_rsrc(fb + rofff[r], fbytes), cbf, fb));
           }
         }
         if constexpr (WY > 1) {
@@ -1234,7 +1236,7 @@ __global__ __launch_bounds__(64 * WY, tb_waves(MODE, sizeof(TS), WY)) void tb_ke
           }
           const TF* fb = (const TF*)adj.fs[fl] + pn * plane;
 #pragma unroll
-          for (int r = 0; r < R; ++r) fv[fl][r] = (M)St<TF>::ld((fb + rofff[r])[colf]);
+          for (int r = 0; r < R; ++r) fv[fl][r] = (M)St<TF>::ld(buf_ld(row_rsrc(fb + rofff[r], fbytes), cbf, fb));
         }
       }
 #pragma unroll
